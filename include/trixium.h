@@ -112,14 +112,15 @@ int trx_gemv_ternary_f32(const uint8_t* rows, int kind, int M, int K, const floa
 /* Multi-position float projection, the batched prefill's GEMM (the float counterpart of
  * model/bitexact.py:121-125 matvec_ternary_rows, one weight pass for many rows): y[r] = W xhat_r
  * for n rows x_r of K floats (xhat = x, or x / rms(x) * norm_w with norm_w != NULL), on the matrix
- * cores. W's rows are decoded to fp16 weights exactly as fastref's fp16 weight cache holds them
- * (model/fastref.py:104-116: (code - 1) * scale, or fp16(q * scale) for Q8) and xhat is split
- * into fp16 hi and lo planes, so each product is fp32-accurate. kind: TRX_KIND_TERNARY,
- * TRX_KIND_TERNARY5 or TRX_KIND_Q8. Epilogues: TRX_EPI_STORE y [n][M]; TRX_EPI_RESID y [n][M] +=;
- * TRX_EPI_SWIGLU (rows [0,F) gate, [F,2F) up) y [n][M/2]. A row of xhat at or above 2^14 in
- * magnitude is scaled by a power of two for the planes and back in the result (exact), so large
- * inputs stay finite. rows must be followed by 16 readable bytes; workspace holds 4*n*(K+1)
- * bytes. */
+ * cores. Ternary rows: xhat enters as five planes of base-32 digits with an exponent per 32 columns,
+ * the trits as they are, and each 128-column sum is multiplied by the group's fp16 scale in float32
+ * ((code - 1) * scale is what model/fastref.py:104-116's fp16 weight cache holds). Q8 rows are
+ * decoded to that cache's fp16(q * scale) and xhat is split into fp16 hi and lo planes. Either way
+ * each product is fp32-accurate. kind: TRX_KIND_TERNARY, TRX_KIND_TERNARY5 or TRX_KIND_Q8.
+ * Epilogues: TRX_EPI_STORE y [n][M]; TRX_EPI_RESID y [n][M] +=;
+ * TRX_EPI_SWIGLU (rows [0,F) gate, [F,2F) up) y [n][M/2]. Inputs of any finite magnitude stay
+ * finite (exponents per block, or per row for Q8: powers of two, exact). rows must be followed by 16
+ * readable bytes; workspace holds 4*n*(K+1) bytes. */
 int trx_gemm_ternary_f32(const uint8_t* rows, int kind, int M, int K, const float* x, int n,
                          const float* norm_w, float eps, float* y, int epilogue, void* workspace,
                          trx_stream_t s);

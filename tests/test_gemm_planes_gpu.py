@@ -1,0 +1,141 @@
+"""The ternary GEMM's digit planes and tile shapes on the GPU (trx_gemm.hip), against float64.
+
+The bound is derived: what the five digits leave of x is at most half an ulp of its 32-column block's
+largest value (2^-24 of it; 2^-105 where the block lies below 2^-80, the smallest exponent), a
+group's ten matrix instructions and the sums over the G groups round in float32 (2^-24 of the partial
+sums each, which the sum of |w x| bounds), and the output adds a few roundings (the RMSNorm's scale,
+the residual). Up to three values 2^7 or more above the rest of their block do not count as its
+largest.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from trixium_amd import _lib, layout as L
+from trixium_amd.bons import encode_rows
+
+pytestmark = pytest.mark.gpu
+
+EPS = 1e-6
+
+
+def _matrix(kind, M, K, rng):
+    codes = rng.integers(0, 4 if kind == L.KIND_TERNARY else 3, (M, K)).astype(np.uint8)
+    sc = rng.uniform(0.01, 0.05, (M, K // 128)).astype(np.float16)
+    w = (codes.astype(np.float64) - 1).reshape(M, -1, 128) * sc.astype(np.float64)[:, :, None]
+    return encode_rows(kind, K, sc, codes), w.reshape(M, K)
+
+
+def _run(rows, kind, M, K, x, gain, epi, y0, work_offset=0):
+    n = x.shape[0]
+    cols = M // 2 if epi == _lib.EPI_SWIGLU else M
+    rb, xb = _lib.DeviceBuffer.from_array(rows), _lib.DeviceBuffer.from_array(x)
+    gb = _lib.DeviceBuffer.from_array(gain) if gain is not None else None
+    yb = _lib.DeviceBuffer.from_array(y0) if y0 is not None else _lib.DeviceBuffer(4 * n * cols)
+    wb = _lib.DeviceBuffer(4 * n * (K + 1) + work_offset)
+    _lib.call("trx_gemm_ternary_f32", rb.ptr, kind, M, K, xb.ptr, n, gb.ptr if gb else None, ctypes.c_float(EPS),
+              yb.ptr, epi, wb.ptr + work_offset, None)
+    _lib.synchronize()
+    return yb.download(np.float32, n * cols).reshape(n, cols).astype(np.float64)
+
+
+def _check(kind, M, K, n, epi, norm, x, rng, work_offset=0, top=None):
+    rows, W = _matrix(kind, M, K, rng)
+    gain = rng.uniform(0.8, 1.2, K).astype(np.float32) if norm else None
+    y0 = rng.standard_normal((n, M)).astype(np.float32) if epi == _lib.EPI_RESID else None
+    v = x.astype(np.float64)
+    r = np.ones((n, 1))
+    if norm:
+        r = 1.0 / np.sqrt(np.mean(v * v, axis=1, keepdims=True) + EPS)
+        v = v * gain.astype(np.float64)
+    G = K // 128
+    # Half 1 of a trit5 group takes its columns one later, so a block spans two of the 32-column runs.
+    if top is None:
+        top = np.abs(v).reshape(n, G, 128).max(axis=2).repeat(128, axis=1)
+    ref, mag = (v @ W.T) * r, (np.abs(v) @ np.abs(W).T) * r
+    err = 2.0**-24 * ((np.maximum(top, 2.0**-81) @ np.abs(W).T) * r + (G + 16) * mag)
+    if epi == _lib.EPI_SWIGLU:
+        F = M // 2
+        g, u = ref[:, :F], ref[:, F:]
+        s = 1 / (1 + np.exp(-np.clip(g, -700, 700)))
+        ref = g * s * u
+        # |silu'| <= 1.1; the exponential and the division add a few float32 roundings of the result.
+        err = 1.1 * err[:, :F] * np.abs(u) + np.abs(g * s) * err[:, F:] + 2.0**-20 * np.abs(ref) + 1e-12
+    elif y0 is not None:
+        ref = ref + y0
+        err = err + 2.0**-23 * np.abs(ref)
+    got = _run(rows, kind, M, K, x, gain, epi, y0, work_offset)
+    worst = float(np.max(np.abs(got - ref) / err))
+    print(f"kind {kind} M {M} K {K} n {n} epi {epi} norm {norm}: worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1.0
+
+
+# Rows and positions around the tiles' edges (32 and 128 positions, 32 to 256 rows), one group (fewer
+# than the waves that split K), groups that eight waves share unevenly, and shapes that take each of
+# the launcher's four tiles on 256 CUs (128 x 256: the last three).
+@pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
+@pytest.mark.parametrize("epi", [_lib.EPI_STORE, _lib.EPI_RESID, _lib.EPI_SWIGLU])
+@pytest.mark.parametrize("M,K,n", [(2, 128, 1), (34, 128, 33), (64, 256, 31), (66, 1152, 32), (1000, 1280, 3),
+                                   (2046, 2048, 65), (4096, 384, 97), (6144, 1152, 200), (2050, 640, 512),
+                                   (12290, 384, 513), (24576, 256, 385), (8190, 128, 1100)])
+def test_tiles_match_float64(kind, epi, M, K, n):
+    rng = np.random.default_rng(M + 7 * K + n + epi)
+    x = (rng.standard_normal((n, K)) * rng.uniform(0.2, 4.0, (n, 1))).astype(np.float32)
+    _check(kind, M, K, n, epi, epi != _lib.EPI_RESID, x, rng)
+
+
+@pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
+def test_magnitudes(kind):
+    """Rows from 1e-30 to 1e30, outliers, zero blocks and denormals: every block has its own exponent."""
+    rng = np.random.default_rng(5)
+    n, K = 40, 768
+    x = rng.standard_normal((n, K))
+    x[:20] *= 10.0 ** np.linspace(-30, 30, 20)[:, None]
+    x[20:30, ::97] *= 1e4
+    x[30, :256] = 0
+    x[31] = 0
+    x[32] *= 1e-42
+    x[33, 5] = 2.0**127
+    _check(kind, 160, K, n, _lib.EPI_STORE, False, x.astype(np.float32), rng)
+
+
+def test_workspace_at_a_dword():
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((37, 512)).astype(np.float32)
+    _check(L.KIND_TERNARY5, 300, 512, 37, _lib.EPI_STORE, True, x, rng, work_offset=4)
+
+
+@pytest.mark.parametrize("n", [5, 300])
+def test_non_finite_rows_stay_apart(n):
+    """A row that holds an infinity or a NaN gives NaN; the other rows are as without it."""
+    rng = np.random.default_rng(8)
+    M, K, kind = 24576 if n == 300 else 512, 384, L.KIND_TERNARY5
+    rows, _ = _matrix(kind, M, K, rng)
+    x = rng.standard_normal((n, K)).astype(np.float32)
+    clean = _run(rows, kind, M, K, x, None, _lib.EPI_STORE, None)
+    x[1, 7], x[3, 200] = np.inf, np.nan
+    got = _run(rows, kind, M, K, x, None, _lib.EPI_STORE, None)
+    bad = np.isin(np.arange(n), (1, 3))
+    assert np.isnan(got[bad]).all()
+    assert np.array_equal(got[~bad], clean[~bad])
+
+
+@pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
+@pytest.mark.parametrize("M,n", [(260, 40), (24576, 400)])
+def test_lone_values_keep_the_rest(kind, M, n):
+    """One to three values 10^4 to 10^30 times the rest, in every place of a group and group of a row in turn: the
+    outputs whose weight there is 0 stay as exact as without it."""
+    rng = np.random.default_rng(M + kind)
+    K = 384 if M > 1000 else 1280
+    x = rng.standard_normal((n, K))
+    rest = 128 * np.abs(x).reshape(n, K // 128, 128).max(axis=2).repeat(128, axis=1)
+    at = (np.arange(n) * 37) % K
+    x[np.arange(n), at] = rng.choice([-1, 1], n) * 10.0 ** rng.uniform(4, 30, n)
+    for step, c, f in ((1, 0, 1.0), (3, 5, 0.3), (6, 9, -0.05)):     # two and three in one block
+        for r in range(0, n, step):
+            col = (at[r] & ~31) + (at[r] + c) % 32
+            x[r, col] = f * x[r, at[r]]
+            rest[r, col] = abs(x[r, at[r]])          # they share a scale of their own
+    _check(kind, M, K, n, _lib.EPI_STORE, False, x.astype(np.float32), rng, top=rest)

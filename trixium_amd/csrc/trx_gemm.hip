@@ -1,0 +1,826 @@
+// The ternary GEMM of several positions on the matrix cores: y[r] = W xhat_r.
+//
+// x enters as five planes of base-32 digits in fp6 (E2M3), W's trits as fp4 (E2M1), so that the
+// products run on v_mfma_scale_f32_32x32x64_f8f6f4 at its fp6/fp4 rate, four times fp16's:
+//   x = 2^u (d0 + d1/32 + d2/32^2 + d3/32^3 + d4/32^4), every digit a whole number in [-16, 16]
+// with one exponent u per position and 32 columns (the largest |x| in [8, 16) * 2^u, but see Lone). E2M3 holds
+// every whole number of eighths up to 16 exactly and E2M1 holds -1, 0, 1 (and 2, the 2-bit code
+// 3) exactly, the plane's power of two is the instruction's block scale, and its fp32 accumulation
+// of such products is exact while a sum fits 24 bits. What is left of x is at most 2^(u - 21): half
+// an ulp of the block's largest value. A group's sum is then multiplied by the group's fp16 scale
+// and added in fp32, so the result is nearer to the exact one than fp32 products added one by one
+// (against float64, K = 4096: 2e-7 of the result's norm; two fp16 planes gave 6e-7).
+// Measured on all CUs (operands in registers, random data): 6.1 PFLOP/s for fp6 x fp4, 3.4 for
+// int8, 1.57 for fp16; with the planes that each needs for fp32-accurate x (5, 3, 2) that is 1.23,
+// 1.14 and 0.79 PFLOP/s, and the int8 planes' sums would need five vector operations per element
+// and group where these need one.
+
+#include "trx_internal.h"
+#include "trx_prefill.h"
+
+namespace trx {
+
+typedef int i32x2_t __attribute__((ext_vector_type(2)));
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+typedef int i32x12_t __attribute__((ext_vector_type(12)));
+typedef unsigned int u32x6_t __attribute__((ext_vector_type(6)));
+typedef float f32x32_t __attribute__((ext_vector_type(32)));
+
+// Digit planes ----------------------------------------------------------------------------------
+//
+// The matrix instruction's operand order: a step takes 64 columns of a 128-column group, lane half
+// h of it 32 of them, position 32 pt + j in lane j. Half h holds the group's columns 64 h .. 64 h +
+// 63, step s its 32 from 32 s on (trit5: half 1 takes columns 65 .. 127 and then 64, whose code
+// shares a byte with half 0's). A position tile's step is 256 P bytes for its P <= 32 positions:
+// eight runs [h][j] of 16-byte pieces that hold a lane's 32 dwords in order, six of each plane (the
+// lowest digit's first), then the block's scales and the fp32 sum of the 32 columns' x^2. Four bytes a column in all, read by 16-byte loads only (per byte, the
+// vector cache is a quarter slower on 8- and 12-byte ones).
+constexpr int kPlanes = 5;
+constexpr int kUMin = -84;             // smallest u: below it values lose bits under 2^-109
+constexpr int kApart = 7;
+// The block scales hold the planes 2^16 down and the weights' scales 2^16 up, so that no group's sum
+// of finite values overflows.
+constexpr int kScaleByte = 110 - 16;
+constexpr float kScaleUp = 65536.f;
+
+template <bool VEC>
+__global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
+  const int lane = threadIdx.x & 63, h = lane >> 5, j = lane & 31;
+  const int st = blockIdx.x * 4 + (threadIdx.x >> 6), pt = blockIdx.y;
+  const int P = min(32, p.R - 32 * pt);
+  if (st >= p.K / 64 || j >= P) return;
+  const int s = st & 1, c0 = 64 * (st & ~1) + 64 * h + 32 * s;
+  const float* xr = p.x + (size_t)(32 * pt + j) * p.ldx + c0;
+  const float* gr = p.norm_w ? p.norm_w + c0 : nullptr;
+  float v[33];
+  if (VEC) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float4 a = ((const float4*)xr)[i];
+      v[4 * i] = a.x;
+      v[4 * i + 1] = a.y;
+      v[4 * i + 2] = a.z;
+      v[4 * i + 3] = a.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 32; ++i) v[i] = xr[i];
+  }
+  const bool turned = p.turned && h;
+  const int ce = turned ? (s ? -32 : 32) : 0;          // the column that ends a turned block
+  v[32] = xr[ce];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) ss += v[i] * v[i];
+  if (gr) {
+    if (VEC) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float4 a = ((const float4*)gr)[i];
+        v[4 * i] *= a.x;
+        v[4 * i + 1] *= a.y;
+        v[4 * i + 2] *= a.z;
+        v[4 * i + 3] *= a.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 32; ++i) v[i] *= gr[i];
+    }
+    v[32] *= gr[ce];
+  }
+  // The block's values, even ones in a, odd ones in b (the conversion interleaves its two sources).
+  f32x16_t a, b;
+  uint32_t top = 0;                                   // the largest magnitude's bits
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    a[i] = turned ? v[2 * i + 1] : v[2 * i];
+    b[i] = turned ? v[2 * i + 2] : v[2 * i + 1];
+    top = max(top, max(__float_as_uint(a[i]) & 0x7FFFFFFFu, __float_as_uint(b[i]) & 0x7FFFFFFFu));
+  }
+  const bool finite = top < 0x7F800000u;
+  // One to three values 2^kApart or more above the rest (see Lone values below): the block's exponent is
+  // the rest's, and they go in 2^-apart times. u from an exponent field E: E - 130.
+  const uint32_t high = top > ((uint32_t)kApart << 23) ? top - ((uint32_t)kApart << 23) : 0;
+  uint32_t rest = 0;
+  int count = 0;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const uint32_t ma = __float_as_uint(a[i]) & 0x7FFFFFFFu, mb = __float_as_uint(b[i]) & 0x7FFFFFFFu;
+    count += (ma >= high) + (mb >= high);
+    rest = max(rest, max(ma >= high ? 0u : ma, mb >= high ? 0u : mb));
+  }
+  int u = max((int)(top >> 23) - 130, kUMin), apart = 0;
+  uint32_t where = 0;
+  if (finite && rest != 0 && count <= 3) {
+    const int un = max((int)(rest >> 23) - 130, kUMin);
+    apart = u - un;
+    u = un;
+    auto lone = [&](float x, int e) {
+      if ((__float_as_uint(x) & 0x7FFFFFFFu) < high) return x;
+      where = where << 5 | (uint32_t)e;
+      return ldexpf(x, -apart);
+    };
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      a[i] = lone(a[i], 2 * i);
+      b[i] = lone(b[i], 2 * i + 1);
+    }
+    for (; count < 3; ++count) where = where << 5 | (where & 31u);
+  }
+  uint8_t* out = p.xp + (size_t)32 * pt * p.K * 4 + (size_t)st * 256 * P;
+  uint4* o = (uint4*)out + h * P + j;
+  uint32_t dw[32];
+#pragma unroll
+  for (int d = 0; d < kPlanes; ++d) {
+    const float sc = __uint_as_float((uint32_t)(u + 3 - 5 * d + 127) << 23);
+    const u32x6_t q = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, sc);
+    // The sources stay live past the conversion: it reads them while it writes its result, and the
+    // compiler may otherwise give both the same registers.
+    asm volatile("" ::"v"(a), "v"(b));
+    if (d + 1 < kPlanes) {
+      const f32x32_t back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
+      asm volatile("" ::"v"(q));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        a[i] -= back[2 * i];
+        b[i] -= back[2 * i + 1];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 6; ++i) dw[6 * (kPlanes - 1 - d) + i] = q[i];
+  }
+  // Byte 0: the block scale of the lowest plane (plane c's is 5 c above); 0xFF, the format's NaN, where a
+  // value is not finite. Byte 1: the lone values' shift; then their three places and bit 31.
+  dw[30] = !finite ? 0xFFu
+                   : (uint32_t)(u + kScaleByte) | (apart > 0 ? (uint32_t)apart << 8 | where << 16 | 0x80000000u : 0u);
+  dw[31] = __float_as_uint(ss);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[2 * P * i] = make_uint4(dw[4 * i], dw[4 * i + 1], dw[4 * i + 2], dw[4 * i + 3]);
+}
+
+int launch_planes(const PlanesParams& p, hipStream_t s) {
+  TRX_CHECK(p.R >= 1 && p.K >= kGroup && p.K % kGroup == 0 && p.ldx >= p.K, TRX_E_INVALID,
+            "prefill input: R=%d K=%d", p.R, p.K);
+  const bool vec = p.ldx % 4 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.norm_w & 15) == 0;
+  const dim3 grid(cdiv(p.K / 64, 4), cdiv(p.R, 32));
+  if (vec) hipLaunchKernelGGL(planes_kernel<true>, grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL(planes_kernel<false>, grid, dim3(256), 0, s, p);
+  TRX_LAUNCHED();
+  return TRX_OK;
+}
+
+// Weights ---------------------------------------------------------------------------------------
+
+// Code byte -> its weights as fp4: a trit5 byte's five nibbles (digit 0 first), a 2-bit byte's four
+// nibbles (twice). E2M1: 0 is 0, 1 is 2, 2 is 4, the sign is bit 3. Every entry is stored once per
+// LDS bank, so the 64 lanes' random bytes never conflict (one copy: 3.3 times the cycles).
+constexpr int kLut = 256 * 32;
+template <int KIND>
+__device__ __forceinline__ void fill_lut(uint32_t* lut) {
+  auto nib = [](int c) { return c == 0 ? 0xAu : c == 1 ? 0u : c == 2 ? 2u : 4u; };
+  const int b = threadIdx.x >> 1, half = threadIdx.x & 1;    // 512 threads
+  uint32_t v = 0;
+  if (KIND == TRX_KIND_TERNARY5) {
+    int r = b;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      v |= nib(r % 3) << (4 * k);
+      r /= 3;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v |= nib((b >> (2 * k)) & 3) << (4 * k);
+    v |= v << 16;
+  }
+  uint4* d = (uint4*)(lut + 32 * b + 16 * half);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) d[i] = make_uint4(v, v, v, v);
+}
+
+// The codes of one row's half group: 16 bytes from a dword boundary, and the group's scale.
+struct Codes {
+  i32x4_t c;
+  uint32_t sc;
+};
+
+template <int KIND>
+struct RowReader {
+  __amdgpu_buffer_rsrc_t rw;
+  uint32_t rbase, code_off;
+  int h;
+  bool valid;
+  __device__ __forceinline__ void init(const GemmParams& p, int r, int half) {
+    valid = r < p.M;
+    rw = make_rsrc(p.W, p.w_bytes);
+    rbase = (uint32_t)(valid ? r : 0) * (uint32_t)p.row_bytes;
+    code_off = (uint32_t)p.code_off;
+    h = half;
+  }
+  __device__ __forceinline__ uint32_t offset(int g) const {
+    return code_off + (KIND == TRX_KIND_TERNARY5 ? 26u * (uint32_t)g + 13u * (uint32_t)h
+                                                 : 32u * (uint32_t)g + 16u * (uint32_t)h);
+  }
+  __device__ __forceinline__ void load(Codes& r, int g) const {
+    r.c = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + (offset(g) & ~3u), 0, 0));
+    r.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
+  }
+  __device__ __forceinline__ float scale(const Codes& r) const {
+    const float v = (float)__builtin_bit_cast(_Float16, (uint16_t)r.sc);
+    return valid ? v * kScaleUp : 0.f;
+  }
+  // The 64 weights of the half group as fp4 in the planes' column order, in parts that a caller can
+  // spread over its other work: begin, look<0 .. 5> (the table reads of byte runs); low() and
+  // high() give the first and the second 32.
+  struct Half {
+    uint32_t d[4], p[KIND == TRX_KIND_TERNARY5 ? 13 : 16];
+  };
+  __device__ __forceinline__ void begin(const Codes& r, int g, Half& v) const {
+    if (KIND == TRX_KIND_TERNARY5) {
+      const uint32_t sh = offset(g) & 3u;
+      v.d[0] = __builtin_amdgcn_alignbyte(r.c[1], r.c[0], sh);
+      v.d[1] = __builtin_amdgcn_alignbyte(r.c[2], r.c[1], sh);
+      v.d[2] = __builtin_amdgcn_alignbyte(r.c[3], r.c[2], sh);
+      v.d[3] = __builtin_amdgcn_alignbyte(0, r.c[3], sh);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v.d[i] = (uint32_t)r.c[i];
+    }
+  }
+  template <int PART>
+  __device__ __forceinline__ void look(Half& v, const uint32_t* t) const {
+    constexpr int lo5[7] = {0, 2, 4, 6, 7, 10, 13}, lo2[7] = {0, 2, 4, 6, 8, 12, 16};
+    constexpr int a = KIND == TRX_KIND_TERNARY5 ? lo5[PART] : lo2[PART];
+    constexpr int b = KIND == TRX_KIND_TERNARY5 ? lo5[PART + 1] : lo2[PART + 1];
+#pragma unroll
+    for (int i = a; i < b; ++i) v.p[i] = t[((v.d[i >> 2] >> (8 * (i & 3))) & 0xFFu) * 32u];
+  }
+  // Holds the uses of the first (second) half's table values behind this point.
+  template <int HALF>
+  __device__ __forceinline__ void ready(Half& v) const {
+    uint32_t* p = v.p;
+    if constexpr (HALF == 0) {
+      asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7]));
+    } else {
+      asm volatile("" : "+v"(p[8]), "+v"(p[9]), "+v"(p[10]), "+v"(p[11]), "+v"(p[12]));
+      if constexpr (KIND == TRX_KIND_TERNARY) asm volatile("" : "+v"(p[13]), "+v"(p[14]), "+v"(p[15]));
+    }
+  }
+  __device__ __forceinline__ i32x4_t low(const Half& v) const {
+    const uint32_t* p = v.p;
+    if (KIND == TRX_KIND_TERNARY5)
+      return i32x4_t{(int)(p[0] | p[1] << 20), (int)(p[1] >> 12 | p[2] << 8 | p[3] << 28), (int)(p[3] >> 4 | p[4] << 16),
+                     (int)(p[4] >> 16 | p[5] << 4 | p[6] << 24)};
+    return i32x4_t{(int)two(p[0], p[1]), (int)two(p[2], p[3]), (int)two(p[4], p[5]), (int)two(p[6], p[7])};
+  }
+  __device__ __forceinline__ i32x4_t high(const Half& v) const {
+    const uint32_t* p = v.p;
+    if (KIND == TRX_KIND_TERNARY5) {
+      // Half 0's last byte ends with column 64, which half 1 takes after its own 63.
+      const auto sw = __builtin_amdgcn_permlane32_swap(p[12], p[12], false, false);
+      const uint32_t end = p[11] >> 4 | p[12] << 16;
+      return i32x4_t{(int)(p[6] >> 8 | p[7] << 12), (int)(p[8] | p[9] << 20), (int)(p[9] >> 12 | p[10] << 8 | p[11] << 28),
+                     (int)(h ? (end & 0x0FFFFFFFu) | (sw[0] >> 16) << 28 : end)};
+    }
+    return i32x4_t{(int)two(p[8], p[9]), (int)two(p[10], p[11]), (int)two(p[12], p[13]), (int)two(p[14], p[15])};
+  }
+  // Two 2-bit bytes' nibbles in one dword (a table entry holds its four nibbles twice).
+  __device__ __forceinline__ static uint32_t two(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+  __device__ __forceinline__ void decode(const Codes& r, int g, const uint32_t* lut, uint32_t (&D)[8]) const {
+    const uint32_t* t = lut + (threadIdx.x & 31);
+    Half v;
+    begin(r, g, v);
+    look<0>(v, t);
+    look<1>(v, t);
+    look<2>(v, t);
+    look<3>(v, t);
+    look<4>(v, t);
+    look<5>(v, t);
+    const i32x4_t a = low(v), b = high(v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      D[i] = (uint32_t)a[i];
+      D[4 + i] = (uint32_t)b[i];
+    }
+  }
+};
+
+// A step's digit planes of one position tile in registers: planes 0 and 1, 2 and 3, and 4 with the
+// block scales (dword 6) and the sum of squares (dword 7).
+struct Planes {
+  i32x12_t c01, c23;
+  i32x8_t c4;
+  template <int C>
+  __device__ __forceinline__ i32x8_t get() const {
+    if constexpr (C == 0) return __builtin_shufflevector(c01, c01, 0, 1, 2, 3, 4, 5, -1, -1);
+    else if constexpr (C == 1) return __builtin_shufflevector(c01, c01, 6, 7, 8, 9, 10, 11, -1, -1);
+    else if constexpr (C == 2) return __builtin_shufflevector(c23, c23, 0, 1, 2, 3, 4, 5, -1, -1);
+    else if constexpr (C == 3) return __builtin_shufflevector(c23, c23, 6, 7, 8, 9, 10, 11, -1, -1);
+    else return c4;
+  }
+  __device__ __forceinline__ uint32_t scales() const { return (uint32_t)c4[6]; }
+  __device__ __forceinline__ float ss() const { return __int_as_float(c4[7]); }
+};
+
+struct PlaneReader {
+  __amdgpu_buffer_rsrc_t r;
+  uint32_t v;                          // this lane's offset in a run of pieces
+  uint32_t P;
+  __device__ __forceinline__ void init(const GemmParams& p, int pt, int lane) {
+    P = (uint32_t)min(32, p.R - 32 * pt);
+    const uint32_t j = min((uint32_t)(lane & 31), P - 1), h = (uint32_t)(lane >> 5);
+    r = make_rsrc(p.xp + (size_t)32 * pt * p.K * 4, 4u * P * (uint32_t)p.K);
+    v = 16u * (h * P + j);
+  }
+  __device__ __forceinline__ uint32_t base(int st) const { return 256u * P * (uint32_t)st; }
+  __device__ __forceinline__ i32x4_t piece(uint32_t base, uint32_t q) const {
+    return __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, base + 32u * P * q, 0));
+  }
+  __device__ __forceinline__ i32x12_t pair(uint32_t base, uint32_t q) const {
+    const i32x4_t a = piece(base, q), b = piece(base, q + 1), c = piece(base, q + 2);
+    return i32x12_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
+  }
+  __device__ __forceinline__ i32x8_t last(uint32_t base) const {
+    const i32x4_t a = piece(base, 6), b = piece(base, 7);
+    return i32x8_t{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  }
+  __device__ __forceinline__ Planes load(int st) const {
+    const uint32_t b = base(st);
+    Planes q;
+    q.c01 = pair(b, 0);
+    q.c23 = pair(b, 3);
+    q.c4 = last(b);
+    return q;
+  }
+};
+
+// acc += plane C of the step's positions times one tile of weights.
+template <int C>
+__device__ __forceinline__ f32x16_t mx(const Planes& q, const i32x4_t& w, const f32x16_t& acc) {
+  const i32x8_t B = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(q.get<C>(), B, acc, 2, 4, 0, (int)(q.scales() + 5u * C), 0,
+                                                          0x7F7F7F7F);
+}
+
+// One plane times NB tiles of weights (independent accumulators), from zero where FIRST.
+template <int C, bool FIRST, int NB>
+__device__ __forceinline__ void mx_plane(const Planes& q, const i32x4_t (&w)[NB], f32x16_t (&t)[NB]) {
+  const f32x16_t zero = {};
+#pragma unroll
+  for (int b = 0; b < NB; ++b) t[b] = mx<C>(q, w[b], FIRST ? zero : t[b]);
+}
+template <bool FIRST, int NB>
+__device__ __forceinline__ void mx_step(const Planes& q, const i32x4_t (&w)[NB], f32x16_t (&t)[NB]) {
+  mx_plane<0, FIRST, NB>(q, w, t);
+  mx_plane<1, false, NB>(q, w, t);
+  mx_plane<2, false, NB>(q, w, t);
+  mx_plane<3, false, NB>(q, w, t);
+  mx_plane<4, false, NB>(q, w, t);
+}
+
+// Weight row of lane j of 32-row tile `tile`: rows in order, or for SwiGLU gate rows f (even tiles)
+// and the matching up rows F + f (odd tiles), f = 32 (tile / 2) + j. M for a row past the end.
+template <int EPI>
+__device__ __forceinline__ int tile_row(int tile, int j, int M) {
+  if (EPI == GM_SWIGLU) {
+    const int F = M / 2, f = 32 * (tile >> 1) + j;
+    return f < F ? ((tile & 1) ? F + f : f) : M;
+  }
+  return min(32 * tile + j, M);
+}
+
+// Lone values. A block's values share an exponent, so a few far above the rest would cost the rest their
+// low bits (a model's massive channels do that; the result's norm would not show it, outputs whose
+// weight there is 0 would). planes_kernel stores such a value v as v' = 2^-apart v at the others'
+// scale. Tiles that met one (a bit of the scales) go over K once more and add v - v' for the steps
+// that hold one: the planes masked to the values' places, once at their scale and once negated at the
+// block's.
+template <int C>
+__device__ __forceinline__ f32x16_t mx_lone(const Planes& q, const i32x4_t& w, f32x16_t acc) {
+  const uint32_t s = q.scales();
+  const bool on = (int)s < 0;
+  const i32x8_t x = q.get<C>();
+  i32x8_t A = {}, N = {};
+#pragma unroll
+  for (int i = 0; i < 6; ++i) {
+    uint32_t mask = 0, sign = 0;                      // a place's six bits, the last its sign
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const int sh = 6 * (int)(s >> (16 + 5 * k) & 31u) - 32 * i;
+      if (on && sh > -6 && sh < 32) mask |= sh >= 0 ? 0x3Fu << sh : 0x3Fu >> -sh;
+      if (on && sh >= -5 && sh < 27) sign |= 1u << (sh + 5);
+    }
+    A[i] = (int)((uint32_t)x[i] & mask);
+    N[i] = A[i] ^ (int)sign;
+  }
+  const i32x8_t B = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
+  const uint32_t s0 = (s & 0xFFu) + 5u * C;
+  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(N, B, acc, 2, 4, 0, (int)s0, 0, 0x7F7F7F7F);
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, acc, 2, 4, 0, (int)(s0 + (on ? s >> 8 & 0xFFu : 0u)), 0,
+                                                          0x7F7F7F7F);
+}
+__device__ __forceinline__ void mx_lone_step(const Planes& q, const i32x4_t& w, f32x16_t& t) {
+  t = mx_lone<0>(q, w, t);
+  t = mx_lone<1>(q, w, t);
+  t = mx_lone<2>(q, w, t);
+  t = mx_lone<3>(q, w, t);
+  t = mx_lone<4>(q, w, t);
+}
+// acc += the lone values of groups g0 .. g1 - 1 times one tile of weights.
+template <int KIND, int EPI>
+__device__ __forceinline__ void add_lone(const GemmParams& p, const PlaneReader& pl, int tile, const uint32_t* lut, int g0,
+                                         int g1, f32x16_t& acc) {
+  const int lane = threadIdx.x & 63;
+  RowReader<KIND> row;
+  row.init(p, tile_row<EPI>(tile, lane & 31, p.M), lane >> 5);
+  for (int g = g0; g < g1; ++g) {
+    const uint32_t s = (uint32_t)pl.piece(pl.base(2 * g), 7)[2] | (uint32_t)pl.piece(pl.base(2 * g + 1), 7)[2];
+    if (!__any((int)s < 0)) continue;
+    Codes codes;
+    row.load(codes, g);
+    uint32_t D[8];
+    row.decode(codes, g, lut, D);
+    f32x16_t t = {};
+    mx_lone_step(pl.load(2 * g), i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]}, t);
+    mx_lone_step(pl.load(2 * g + 1), i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]}, t);
+    const float sc = row.scale(codes);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = fmaf(t[e], sc, acc[e]);
+  }
+}
+
+// Block b of nx weight tiles x ny position tiles. Blocks go to the 8 XCDs in turn; each XCD takes
+// one run of an order that walks panels of 8 weight tiles position by position, so that the blocks
+// which share an L2 at a time share their weights and their positions.
+__device__ __forceinline__ void tile_of_block(int b, int nx, int ny, int& x, int& y) {
+  const int total = nx * ny, q = total / 8, rem = total % 8, xcd = b % 8, k = b / 8;
+  const int L = xcd < rem ? xcd * (q + 1) + k : rem * (q + 1) + (xcd - rem) * q + k;
+  const int full = nx / 8 * 8;
+  if (L < full * ny) {
+    const int panel = L / (8 * ny), r = L - panel * 8 * ny;
+    x = 8 * panel + r % 8;
+    y = r / 8;
+  } else {
+    const int w = nx - full, r = L - full * ny;
+    x = full + r % w;
+    y = r / w;
+  }
+}
+
+constexpr int kGmThreads = 512;
+
+// Large products: a block takes 128 positions x 256 weight rows. Wave w holds position tile w % 4
+// and weight tiles 4 (w / 4) .. + 3 (64 accumulator registers, 64 more for a group's sums); it loads
+// its positions' planes straight into registers (the operand order makes each load contiguous), most
+// of a group ahead of their use, and decodes one of the block's eight weight tiles per group into
+// LDS for all waves, two buffers, one barrier a group.
+// A wave alone issues a vector operation every 6 cycles beside the matrix unit's 32-cycle products,
+// so all of a group's vector work (the last group's sums into the accumulators, the next group's
+// decode) is laid out between the products: 20 slots of two products and about ten operations.
+template <int KIND, int EPI>
+__global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
+  __shared__ __align__(16) uint32_t lut[kLut];
+  __shared__ __align__(16) i32x4_t bs[2][8][2][64];
+  __shared__ float wsc[2][256];
+  __shared__ float rsx[128];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, j = lane & 31;
+  const int pw = w & 3, ww = w >> 2;
+  int bx, by;
+  tile_of_block(blockIdx.x, p.nx, p.ny, bx, by);
+  const int G = p.K / kGroup, npt = (p.R + 31) / 32;
+  const int pt = min(4 * by + pw, npt - 1);           // a tile past the last repeats it, unstored
+  const bool live = 4 * by + pw < npt;
+
+  RowReader<KIND> row;
+  row.init(p, tile_row<EPI>(8 * bx + w, j, p.M), h);
+  PlaneReader pl;
+  pl.init(p, pt, lane);
+  Codes codes, next;                                  // the next group's, and the one after
+  row.load(codes, 0);
+  Planes q0 = pl.load(0), q1 = pl.load(1);
+  fill_lut<KIND>(lut);
+  __syncthreads();
+  {
+    uint32_t D[8];
+    row.decode(codes, 0, lut, D);
+    bs[0][w][0][lane] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
+    bs[0][w][1][lane] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
+    wsc[0][32 * w + j] = row.scale(codes);
+    row.load(codes, min(1, G - 1));
+    row.load(next, min(2, G - 1));
+  }
+  __syncthreads();
+  f32x16_t acc0 = {}, acc1 = {}, acc2 = {}, acc3 = {}, t0 = {}, t1 = {}, t2 = {}, t3 = {};
+  float ss = 0.f, s2 = 0.f, s3 = 0.f;
+  uint32_t lone = 0;
+  const i32x4_t (*fr)[2][64] = &bs[0][4 * ww];        // this wave's four tiles
+  i32x4_t x0 = fr[0][0][lane], x1 = fr[1][0][lane], y0, y1;
+  const f32x16_t zero = {};
+#define TRX_FMA(A, T, S, E0)                                                \
+  _Pragma("unroll") for (int e = E0; e < E0 + 8; ++e) A[e] = fmaf(T[e], S, A[e])
+#define TRX_SLOT(C, Q, TA, TB, XA, XB, CA, CB) \
+  TA = mx<C>(Q, XA, CA);                       \
+  TB = mx<C>(Q, XB, CB);                       \
+  asm volatile("" : "+v"(TA), "+v"(TB) : : "memory")
+#define TRX_PIN1(A) asm volatile("" : "+v"(A))
+  for (int g = 0; g < G; ++g) {
+    const int buf = g & 1, gn = min(g + 1, G - 1);
+    const uint32_t n0 = pl.base(2 * gn), n1 = pl.base(2 * gn + 1);
+    const uint32_t* lt = lut + (lane & 31);
+    fr = &bs[buf][4 * ww];
+    lone |= q0.scales() | q1.scales();
+    // Step 0, tiles 0 and 1; the last group's tiles 2 and 3 into their accumulators.
+    y0 = fr[2][0][lane];
+    y1 = fr[3][0][lane];
+    ss += q0.ss();
+    ss += q1.ss();
+    TRX_SLOT(0, q0, t0, t1, x0, x1, zero, zero);
+    TRX_SLOT(1, q0, t0, t1, x0, x1, t0, t1);
+    TRX_FMA(acc2, t2, s2, 0);
+    TRX_PIN1(acc2);
+    TRX_SLOT(2, q0, t0, t1, x0, x1, t0, t1);
+    TRX_FMA(acc2, t2, s2, 8);
+    TRX_PIN1(acc2);
+    TRX_SLOT(3, q0, t0, t1, x0, x1, t0, t1);
+    TRX_FMA(acc3, t3, s3, 0);
+    TRX_PIN1(acc3);
+    TRX_SLOT(4, q0, t0, t1, x0, x1, t0, t1);
+    TRX_FMA(acc3, t3, s3, 8);
+    TRX_PIN1(acc3);
+    // Step 0, tiles 2 and 3; the planes' registers take the next group's; the codes' first half.
+    typename RowReader<KIND>::Half hv;
+    row.begin(codes, gn, hv);
+    x0 = fr[0][1][lane];
+    x1 = fr[1][1][lane];
+    TRX_SLOT(0, q0, t2, t3, y0, y1, zero, zero);
+    row.template look<0>(hv, lt);
+    TRX_SLOT(1, q0, t2, t3, y0, y1, t2, t3);
+    q0.c01 = pl.pair(n0, 0);
+    row.template look<1>(hv, lt);
+    TRX_SLOT(2, q0, t2, t3, y0, y1, t2, t3);
+    row.template look<2>(hv, lt);
+    TRX_SLOT(3, q0, t2, t3, y0, y1, t2, t3);
+    q0.c23 = pl.pair(n0, 3);
+    row.template look<3>(hv, lt);
+    TRX_SLOT(4, q0, t2, t3, y0, y1, t2, t3);
+    q0.c4 = pl.last(n0);
+    i32x4_t D0 = row.low(hv);
+    TRX_PIN1(D0);
+    // Step 1, tiles 0 and 1; the codes' second half.
+    y0 = fr[2][1][lane];
+    y1 = fr[3][1][lane];
+    TRX_SLOT(0, q1, t0, t1, x0, x1, t0, t1);
+    bs[buf ^ 1][w][0][lane] = D0;
+    row.template look<4>(hv, lt);
+    TRX_SLOT(1, q1, t0, t1, x0, x1, t0, t1);
+    row.template look<5>(hv, lt);
+    const float s0 = wsc[buf][32 * (4 * ww) + j], s1 = wsc[buf][32 * (4 * ww + 1) + j];
+    TRX_SLOT(2, q1, t0, t1, x0, x1, t0, t1);
+    s2 = wsc[buf][32 * (4 * ww + 2) + j];
+    s3 = wsc[buf][32 * (4 * ww + 3) + j];
+    wsc[buf ^ 1][32 * w + j] = row.scale(codes);
+    TRX_SLOT(3, q1, t0, t1, x0, x1, t0, t1);
+    i32x4_t D1 = row.high(hv);
+    TRX_PIN1(D1);
+    TRX_SLOT(4, q1, t0, t1, x0, x1, t0, t1);
+    bs[buf ^ 1][w][1][lane] = D1;
+    codes = next;
+    row.load(next, min(g + 3, G - 1));
+    // Step 1, tiles 2 and 3; after the barrier the next group's first weights.
+    TRX_SLOT(0, q1, t2, t3, y0, y1, t2, t3);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    fr = &bs[buf ^ 1][4 * ww];
+    x0 = fr[0][0][lane];
+    x1 = fr[1][0][lane];
+    TRX_SLOT(1, q1, t2, t3, y0, y1, t2, t3);
+    q1.c01 = pl.pair(n1, 0);
+    TRX_FMA(acc0, t0, s0, 0);
+    TRX_PIN1(acc0);
+    TRX_SLOT(2, q1, t2, t3, y0, y1, t2, t3);
+    TRX_FMA(acc0, t0, s0, 8);
+    TRX_PIN1(acc0);
+    TRX_SLOT(3, q1, t2, t3, y0, y1, t2, t3);
+    q1.c23 = pl.pair(n1, 3);
+    TRX_FMA(acc1, t1, s1, 0);
+    TRX_PIN1(acc1);
+    TRX_SLOT(4, q1, t2, t3, y0, y1, t2, t3);
+    q1.c4 = pl.last(n1);
+    TRX_FMA(acc1, t1, s1, 8);
+    TRX_PIN1(acc1);
+  }
+  TRX_FMA(acc2, t2, s2, 0);
+  TRX_FMA(acc2, t2, s2, 8);
+  TRX_FMA(acc3, t3, s3, 0);
+  TRX_FMA(acc3, t3, s3, 8);
+  if (__any((int)lone < 0)) {
+    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww, lut, 0, G, acc0);
+    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 1, lut, 0, G, acc1);
+    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 2, lut, 0, G, acc2);
+    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 3, lut, 0, G, acc3);
+  }
+#undef TRX_FMA
+#undef TRX_SLOT
+#undef TRX_PIN1
+
+  // Accumulator e of lane l holds position i = 8 (e / 4) + 4 (l / 32) + e % 4, weight row l % 32.
+  if (ww == 0) {
+    ss += __shfl_xor(ss, 32, 64);
+    if (h == 0) rsx[32 * pw + j] = p.norm ? 1.0f / sqrtf(ss / (float)p.K + p.eps) : 1.f;
+  }
+  __syncthreads();
+  if (!live) return;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int i = 8 * (e >> 2) + 4 * h + (e & 3), r = 32 * pt + i;
+    if (r >= p.R) continue;
+    const float rs = rsx[32 * pw + i];
+    float* yr = p.y + (size_t)r * p.ldy;
+    const float v[4] = {acc0[e] * rs, acc1[e] * rs, acc2[e] * rs, acc3[e] * rs};
+    if (EPI == GM_SWIGLU) {
+#pragma unroll
+      for (int b = 0; b < 4; b += 2) {
+        const int f = 32 * ((8 * bx + 4 * ww + b) >> 1) + j;
+        if (f < p.M / 2) yr[f] = silu(v[b]) * v[b + 1];
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int m = 32 * (8 * bx + 4 * ww + b) + j;
+        if (m < p.M) {
+          if (EPI == GM_RESID) yr[m] += v[b];
+          else yr[m] = v[b];
+        }
+      }
+    }
+  }
+}
+
+// Products whose grid of large tiles would leave the chip idle: a block takes 32 positions x 32 NB
+// weight rows and its eight waves split K, each decoding its own groups' weights in registers; the
+// waves' sums are added through LDS in wave order.
+template <int KIND, int EPI, int NB>
+__global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p) {
+  constexpr int PT = NB < 2 ? 1 : 2;                  // tiles reduced at a time
+  constexpr int kRed = 8 * PT * 1024;
+  __shared__ __align__(16) uint32_t sm[kRed > kLut ? kRed : kLut];
+  __shared__ float ssx[8][32];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, j = lane & 31;
+  int bx, pt;
+  tile_of_block(blockIdx.x, p.nx, p.ny, bx, pt);
+  const int G = p.K / kGroup, g0 = G * w / 8, g1 = G * (w + 1) / 8;
+  RowReader<KIND> row[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) row[b].init(p, tile_row<EPI>(NB * bx + b, j, p.M), h);
+  PlaneReader pl;
+  pl.init(p, pt, lane);
+  Codes codes[NB];
+  const int gf = min(g0, G - 1);
+#pragma unroll
+  for (int b = 0; b < NB; ++b) row[b].load(codes[b], gf);
+  Planes q0 = pl.load(2 * gf), q1 = pl.load(2 * gf + 1);
+  fill_lut<KIND>(sm);
+  __syncthreads();
+  f32x16_t acc[NB] = {};
+  float ss = 0.f;
+  uint32_t lone = 0;
+  for (int g = g0; g < g1; ++g) {
+    i32x4_t b0[NB], b1[NB];
+    float sc[NB];
+    const int gn = min(g + 1, g1 - 1);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      uint32_t D[8];
+      row[b].decode(codes[b], g, sm, D);
+      b0[b] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
+      b1[b] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
+      sc[b] = row[b].scale(codes[b]);
+      row[b].load(codes[b], gn);
+    }
+    lone |= q0.scales() | q1.scales();
+    f32x16_t t[NB];
+    mx_step<true, NB>(q0, b0, t);
+    ss += q0.ss();
+    q0 = pl.load(2 * gn);
+    mx_step<false, NB>(q1, b1, t);
+    ss += q1.ss();
+    q1 = pl.load(2 * gn + 1);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[b][e] = fmaf(t[b][e], sc[b], acc[b][e]);
+  }
+  if (__any((int)lone < 0)) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) add_lone<KIND, EPI>(p, pl, NB * bx + b, sm, g0, g1, acc[b]);
+  }
+  ss += __shfl_xor(ss, 32, 64);
+  if (h == 0) ssx[w][j] = ss;
+  float4* red = (float4*)sm;                          // [wave][tile][e / 4][lane]
+#pragma unroll
+  for (int b0 = 0; b0 < NB; b0 += PT) {
+    __syncthreads();                                  // the table's or the last pass's reads are done
+#pragma unroll
+    for (int b = 0; b < PT; ++b)
+#pragma unroll
+      for (int e4 = 0; e4 < 4; ++e4)
+        red[((w * PT + b) * 4 + e4) * 64 + lane] = make_float4(acc[b0 + b][4 * e4], acc[b0 + b][4 * e4 + 1],
+                                                               acc[b0 + b][4 * e4 + 2], acc[b0 + b][4 * e4 + 3]);
+    __syncthreads();
+    constexpr int per = EPI == GM_SWIGLU ? 1 : PT;    // output tiles of the pass
+    if (w >= 4 * per) continue;
+    const int tb = w >> 2, e4 = w & 3;
+    float4 v[2];
+#pragma unroll
+    for (int u = 0; u < (EPI == GM_SWIGLU ? 2 : 1); ++u) {
+      v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      const int b = EPI == GM_SWIGLU ? u : tb;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float4 a = red[((k * PT + b) * 4 + e4) * 64 + lane];
+        v[u] = make_float4(v[u].x + a.x, v[u].y + a.y, v[u].z + a.z, v[u].w + a.w);
+      }
+    }
+    const int tile = NB * bx + b0 + tb;
+    const int m = EPI == GM_SWIGLU ? 32 * (tile >> 1) + j : 32 * tile + j;
+    const float a0[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, a1[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int i = 8 * e4 + 4 * h + k, r = 32 * pt + i;
+      if (r >= p.R || m >= (EPI == GM_SWIGLU ? p.M / 2 : p.M)) continue;
+      float rs = 1.f;
+      if (p.norm) {
+        float tot = 0.f;
+#pragma unroll
+        for (int z = 0; z < 8; ++z) tot += ssx[z][i];
+        rs = 1.0f / sqrtf(tot / (float)p.K + p.eps);
+      }
+      float* y = p.y + (size_t)r * p.ldy + m;
+      if (EPI == GM_SWIGLU) *y = silu(a0[k] * rs) * (a1[k] * rs);
+      else if (EPI == GM_RESID) *y += a0[k] * rs;
+      else *y = a0[k] * rs;
+    }
+  }
+}
+
+template <int KIND, int EPI>
+static void gemm_ternary_kind(GemmParams& p, int nb, hipStream_t s) {
+  const int tiles = EPI == GM_SWIGLU ? 2 * cdiv(p.M / 2, 32) : cdiv(p.M, 32);
+  if (nb == 0) {
+    p.nx = cdiv(tiles, 8);
+    p.ny = cdiv(p.R, 128);
+    hipLaunchKernelGGL((gemm_kernel<KIND, EPI>), dim3(p.nx * p.ny), dim3(kGmThreads), 0, s, p);
+    return;
+  }
+  p.nx = cdiv(tiles, nb);
+  p.ny = cdiv(p.R, 32);
+  const dim3 grid(p.nx * p.ny);
+  if (nb == 4) hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 4>), grid, dim3(kGmThreads), 0, s, p);
+  else if (nb == 2) hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 2>), grid, dim3(kGmThreads), 0, s, p);
+  else hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI == GM_SWIGLU ? GM_STORE : EPI, 1>), grid, dim3(kGmThreads), 0, s, p);
+}
+
+template <int KIND>
+static void gemm_ternary_epi(GemmParams& p, int nb, hipStream_t s) {
+  if (p.epi == GM_SWIGLU) gemm_ternary_kind<KIND, GM_SWIGLU>(p, nb, s);
+  else if (p.epi == GM_RESID) gemm_ternary_kind<KIND, GM_RESID>(p, nb, s);
+  else gemm_ternary_kind<KIND, GM_STORE>(p, nb, s);
+}
+
+int launch_gemm_ternary(const GemmParams& params, hipStream_t s) {
+  GemmParams p = params;
+  TRX_CHECK(p.kind == TRX_KIND_TERNARY || p.kind == TRX_KIND_TERNARY5, TRX_E_INVALID,
+            "prefill GEMM: weight kind %d unsupported", p.kind);
+  TRX_CHECK(p.M >= 1 && p.K >= kGroup && p.K % kGroup == 0 && p.R >= 1, TRX_E_INVALID,
+            "prefill GEMM: M=%d K=%d R=%d", p.M, p.K, p.R);
+  TRX_CHECK(p.epi != GM_SWIGLU || p.M % 2 == 0, TRX_E_INVALID, "prefill GEMM: SwiGLU needs an even M");
+  TRX_CHECK((size_t)p.M * p.row_bytes < (1ull << 32) && (size_t)p.M * p.row_bytes + 16 <= p.w_bytes, TRX_E_INVALID,
+            "prefill GEMM: operands too large");
+  int cus = 0, dev = 0;
+  TRX_HIP(hipGetDevice(&dev));
+  TRX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  // The tile with the least estimated time: rounds of blocks over the CUs times a round's length, in
+  // us per 128 columns as measured at full rounds: 2.75 for the 128 x 256 tiles, 0.72, 0.46 and 0.36
+  // for the K-split tiles of 32 x 128, 64 and 32 (of 8, 4, 2 and 1 times the smallest's products per
+  // wave's step: small tiles fill the chip on short prompts and narrow matrices only. 512 positions
+  // of a 2048 x 2048 matrix: 61 us in 32 large tiles, 25, 28 and 33 in 256, 512 and 1024 split ones;
+  // 2048 of a 24576 x 4096: 530 us against 1036).
+  const int tiles = p.epi == GM_SWIGLU ? 2 * cdiv(p.M / 2, 32) : cdiv(p.M, 32), npt = cdiv(p.R, 32);
+  const float len[4] = {2.75f, 0.72f, 0.46f, 0.36f};
+  const int per[4] = {8, 4, 2, 1};
+  int nb = 0;
+  float best = 0.f;
+  for (int i = 0; i < (p.epi == GM_SWIGLU ? 3 : 4); ++i) {
+    const long long blocks = (long long)cdiv(tiles, per[i]) * (i == 0 ? cdiv(p.R, 128) : npt);
+    const float t = len[i] * (float)((blocks + cus - 1) / cus);
+    if (i == 0 || t < best) {
+      best = t;
+      nb = i == 0 ? 0 : per[i];
+    }
+  }
+  if (p.kind == TRX_KIND_TERNARY5) gemm_ternary_epi<TRX_KIND_TERNARY5>(p, nb, s);
+  else gemm_ternary_epi<TRX_KIND_TERNARY>(p, nb, s);
+  TRX_LAUNCHED();
+  return TRX_OK;
+}
+
+}  // namespace trx

@@ -118,7 +118,10 @@ struct Model {
   // that leaves most CUs idle, as the DeltaNet beta|alpha rows': up to 16 parts of 128 columns).
   float* pf_part = nullptr;
   _Float16 *pf_h = nullptr, *pf_l = nullptr;
-  float* pf_xs = nullptr;                          // [pf_rows] row scales of the input planes
+  float* pf_xs = nullptr;                          // [pf_rows] row scales of the fp16 planes
+  uint8_t* pf_planes = nullptr;                    // the ternary GEMM's digit planes
+  bool pf_norm = false;                            // they wait for 1 / rms(x)
+  float* pf_rot = nullptr;                         // a rotated model's rotated input rows
   float* pf_rs = nullptr;                          // [pf_rows] a rotated input's 1/rms per row
   int host_n_fed = 0, host_head_from = 0;          // host copies of the control words
   hipGraph_t graph = nullptr;
@@ -826,12 +829,49 @@ static int run_step(Model& m, hipStream_t s) {
 
 // Batched prefill of positions p0 .. p0 + R - 1 --------------------------------------------------
 
-// The input planes of a projection of width K: RMSNorm (norm_w), and a rotated model's rotation of
-// that width unless `plain` (the DeltaNet beta/alpha take the unrotated input).
-static int pf_prep(Model& m, const float* x, int ldx, int K, int R, const float* norm_w, bool plain, hipStream_t s) {
-  PrepParams pp = {};
+// The digit planes of a ternary projection's input of width K: the RMSNorm's gain (norm_w), and a
+// rotated model's rotation of that width.
+static int pf_prep(Model& m, const float* x, int ldx, int K, int R, const float* norm_w, hipStream_t s) {
+  PlanesParams pp = {};
   pp.x = x;
   pp.ldx = ldx;
+  pp.K = K;
+  pp.R = R;
+  pp.norm_w = norm_w;
+  pp.turned = m.cfg.weight_kind == TRX_KIND_TERNARY5;
+  pp.xp = m.pf_planes;
+  m.pf_norm = norm_w != nullptr;
+  if (m.cfg.hadamard_block) {
+    int wi = 0, rc;
+    while (wi < 4 && m.cfg.hadamard_widths[wi] != K) ++wi;
+    TRX_CHECK(wi < 4, TRX_E_INVALID, "rotated model: no rotation for input width %d", K);
+    RotateRowsParams rp = {};
+    rp.x = x;
+    rp.ldx = ldx;
+    rp.K = K;
+    rp.R = R;
+    rp.norm_w = norm_w;
+    rp.eps = m.cfg.rms_eps;
+    rp.signs = PF(m, TRX_ROLE_HADAMARD, wi);
+    rp.B = m.cfg.hadamard_block;
+    rp.scale = m.cfg.hadamard_scale;
+    rp.rs = m.pf_rs;
+    rp.out = m.pf_rot;
+    if ((rc = launch_rotate_rows(rp, s))) return rc;
+    pp.x = m.pf_rot;
+    pp.ldx = K;
+    pp.norm_w = nullptr;
+    m.pf_norm = false;
+  }
+  return launch_planes(pp, s);
+}
+
+// The fp16 planes of a Q8 projection's input (the DeltaNet beta|alpha, which take the normed input
+// unrotated).
+static int pf_prep_q8(Model& m, const float* x, int K, int R, const float* norm_w, hipStream_t s) {
+  PrepParams pp = {};
+  pp.x = x;
+  pp.ldx = K;
   pp.K = K;
   pp.R = R;
   pp.norm_w = norm_w;
@@ -839,19 +879,10 @@ static int pf_prep(Model& m, const float* x, int ldx, int K, int R, const float*
   pp.xh = m.pf_h;
   pp.xl = m.pf_l;
   pp.xs = m.pf_xs;
-  pp.rs = m.pf_rs;
-  if (m.cfg.hadamard_block && !plain) {
-    int wi = 0;
-    while (wi < 4 && m.cfg.hadamard_widths[wi] != K) ++wi;
-    TRX_CHECK(wi < 4, TRX_E_INVALID, "rotated model: no rotation for input width %d", K);
-    pp.signs = PF(m, TRX_ROLE_HADAMARD, wi);
-    pp.B = m.cfg.hadamard_block;
-    pp.scale = m.cfg.hadamard_scale;
-  }
   return launch_prep(pp, s);
 }
 
-// One GEMM over the planes pf_prep left: W's rows (role, layer; the fused group starting there).
+// One GEMM over the planes pf_prep (or pf_prep_q8) left: W's rows (role, layer; the fused group starting there).
 static int pf_gemm(Model& m, int role, int l, int kind, int M, int K, int R, int epi, float* y, int ldy,
                    hipStream_t s) {
   const Tensor& t = T(m, role, l);
@@ -866,6 +897,9 @@ static int pf_gemm(Model& m, int role, int l, int kind, int M, int K, int R, int
   g.xh = m.pf_h;
   g.xl = m.pf_l;
   g.xs = m.pf_xs;
+  g.xp = m.pf_planes;
+  g.norm = m.pf_norm;
+  g.eps = m.cfg.rms_eps;
   g.R = R;
   g.epi = epi;
   g.y = y;
@@ -901,9 +935,11 @@ static int pf_alloc(Model& m, int R) {
   // (buffer, bytes per row) of every prefill buffer.
   const std::vector<std::pair<void**, size_t>> bufs = {
       {(void**)&m.pf_x, (size_t)E * 4},
-      {(void**)&m.pf_h, (size_t)kmax * 2},
-      {(void**)&m.pf_l, (size_t)kmax * 2},
-      {(void**)&m.pf_xs, 4},
+      {(void**)&m.pf_planes, (size_t)kmax * 4},
+      {(void**)&m.pf_rot, c.hadamard_block ? (size_t)kmax * 4 : 0},
+      {(void**)&m.pf_h, m.n_dn ? (size_t)E * 2 : 0},
+      {(void**)&m.pf_l, m.n_dn ? (size_t)E * 2 : 0},
+      {(void**)&m.pf_xs, m.n_dn ? (size_t)4 : 0},
       {(void**)&m.pf_rs, 4},
       {(void**)&m.pf_qkv, (size_t)io * 4},
       {(void**)&m.pf_att, (size_t)att * 4},
@@ -912,7 +948,7 @@ static int pf_alloc(Model& m, int R) {
       {(void**)&m.pf_ba, m.n_dn ? (size_t)2 * c.dn_num_v_heads * 4 : 0},
       {(void**)&m.pf_conv, m.n_dn ? (size_t)C * 4 : 0},
       {(void**)&m.pf_oraw, m.n_dn ? (size_t)nvh * 4 : 0},
-      {(void**)&m.pf_part, (size_t)kPfPartRow * 4}};
+      {(void**)&m.pf_part, m.n_dn ? (size_t)kPfPartRow * 4 : 0}};
   int rc;
   if (m.pf_rows > 0) {
     TRX_HIP(hipStreamSynchronize(m.stream));
@@ -961,9 +997,9 @@ static int run_prefill(Model& m, int p0, int R, hipStream_t s) {
       const int nq = c.dn_num_k_heads * c.dn_k_head_dim, nvh = c.dn_num_v_heads * c.dn_v_head_dim;
       const int C = 2 * nq + nvh, nv = c.dn_num_v_heads;
       // beta|alpha (Q8) from the unrotated normed input, then qkv|z.
-      if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), true, s))) return rc;
+      if ((rc = pf_prep_q8(m, m.pf_x, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), s))) return rc;
       if ((rc = pf_gemm(m, TRX_ROLE_SSM_BETA, l, TRX_KIND_Q8, 2 * nv, E, R, GM_STORE, m.pf_ba, 2 * nv, s))) return rc;
-      if (c.hadamard_block && (rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), false, s))) return rc;
+      if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), s))) return rc;
       if ((rc = pf_gemm(m, TRX_ROLE_ATTN_QKV, l, wk, C + nvh, E, R, GM_STORE, m.pf_qkv, C + nvh, s))) return rc;
       DnRowsParams dp = {};
       dp.io = m.pf_qkv;
@@ -988,11 +1024,11 @@ static int run_prefill(Model& m, int p0, int R, hipStream_t s) {
       dp.hv = c.dn_v_head_dim;
       dp.eps = c.rms_eps;
       if ((rc = launch_dn_rows(dp, s))) return rc;
-      if ((rc = pf_prep(m, m.pf_att, nvh, nvh, R, nullptr, false, s))) return rc;
+      if ((rc = pf_prep(m, m.pf_att, nvh, nvh, R, nullptr, s))) return rc;
       if ((rc = pf_gemm(m, TRX_ROLE_SSM_OUT, l, wk, E, nvh, R, GM_RESID, m.pf_x, E, s))) return rc;
     } else {
       const int M = qrows + 2 * kvrows;
-      if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), false, s))) return rc;
+      if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_ATTN_NORM, l), s))) return rc;
       if ((rc = pf_gemm(m, TRX_ROLE_ATTN_Q, l, wk, M, E, R, GM_STORE, m.pf_qkv, M, s))) return rc;
       const size_t per = (size_t)c.n_kv_head * c.max_ctx * hd;
       RopeKvParams rp = {};
@@ -1031,12 +1067,12 @@ static int run_prefill(Model& m, int p0, int R, hipStream_t s) {
       ap.max_ctx = c.max_ctx;
       ap.gated = c.attn_gated;
       if ((rc = launch_attn_prefill(ap, s))) return rc;
-      if ((rc = pf_prep(m, m.pf_att, c.n_head * hd, c.n_head * hd, R, nullptr, false, s))) return rc;
+      if ((rc = pf_prep(m, m.pf_att, c.n_head * hd, c.n_head * hd, R, nullptr, s))) return rc;
       if ((rc = pf_gemm(m, TRX_ROLE_ATTN_OUT, l, wk, E, c.n_head * hd, R, GM_RESID, m.pf_x, E, s))) return rc;
     }
-    if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_FFN_NORM, l), false, s))) return rc;
+    if ((rc = pf_prep(m, m.pf_x, E, E, R, PF(m, TRX_ROLE_FFN_NORM, l), s))) return rc;
     if ((rc = pf_gemm(m, TRX_ROLE_FFN_GATE, l, wk, 2 * F, E, R, GM_SWIGLU, m.pf_act, F, s))) return rc;
-    if ((rc = pf_prep(m, m.pf_act, F, F, R, nullptr, false, s))) return rc;
+    if ((rc = pf_prep(m, m.pf_act, F, F, R, nullptr, s))) return rc;
     if ((rc = pf_gemm(m, TRX_ROLE_FFN_DOWN, l, wk, E, F, R, GM_RESID, m.pf_x, E, s))) return rc;
   }
   // The last position's residual is readable as the last forward's (TRX_READ_RESIDUAL), and the

@@ -7,53 +7,79 @@
 
 namespace trx {
 
-// Ternary (or Q8) GEMM on the matrix cores: Y[r][m] = sum_k X[r][k] W[m][k] for R positions.
-// W is read as stored (BONS row packets, M rows of row_bytes) and decoded per 128-column group
-// into LDS as fp16 weights (code - 1) * scale (2-bit, trit5) or fp16(q * scale) (Q8), which are
-// exactly fastref's fp16 weight cache (model/fastref.py:104-116). X comes as two fp16 planes,
-// xh = fp16(x') and xl = fp16(x' - xh) of x' = x / xs[r], so that each product of the fp32
-// accumulation sees x to ~22 bits (the result is within float32 rounding of the fp32 product);
-// xs[r] is a power of two that keeps row r's planes finite (1 for rows below 2^14), multiplied
-// back in the epilogue.
+// GEMM on the matrix cores: Y[r][m] = sum_k X[r][k] W[m][k] for R positions, W read as stored
+// (BONS row packets, M rows of row_bytes). Ternary rows (trx_gemm.hip): X comes as the digit planes
+// of launch_planes; with `norm` they hold x * gain and the sums are scaled by 1 / rms(x) here, from
+// the planes' sums of x^2. Q8 rows (trx_prefill.hip): decoded to fp16(q * scale), which is exactly
+// fastref's fp16 weight cache (model/fastref.py:104-116), and X comes as the two fp16 planes of
+// launch_prep, xh = fp16(x') and xl = fp16(x' - xh) of x' = x / xs[r], so that each product of the
+// fp32 accumulation sees x to ~22 bits; xs[r] is a power of two that keeps row r's planes finite (1
+// for rows below 2^14), multiplied back in the epilogue.
 enum { GM_STORE = 0, GM_RESID = 1, GM_SWIGLU = 2 };
 struct GemmParams {
   const uint8_t* W;        // row packets
   uint32_t w_bytes;        // bytes readable from W (the buffer descriptor's range)
   int kind;                // TRX_KIND_TERNARY, TRX_KIND_TERNARY5 or TRX_KIND_Q8
   int M, K, row_bytes, code_off;
-  const _Float16* xh;      // [R][K]
+  const uint8_t* xp;       // ternary: digit planes, 4 R K bytes
+  int norm;
+  float eps;
+  const _Float16* xh;      // Q8: [R][K]
   const _Float16* xl;      // [R][K]
   const float* xs;         // [R] row scales (powers of two)
   int R;
   int epi;
   float* y;                // GM_STORE: y[r*ldy + m] = acc; GM_RESID: y[r*ldy + m] += acc;
   int ldy;                 // GM_SWIGLU (W = [gate; up], M = 2F): y[r*ldy + f] = silu(g[f]) * u[f]
-  // GM_STORE with few blocks (a small M): with part != null K may be split over up to 16 parts
+  // Q8, GM_STORE with few blocks (a small M): with part != null K may be split over up to 16 parts
   // whose sums go to part[z][R][ldy] (part_floats of room) and are then added in part order.
   float* part;
   size_t part_floats;
+  int nx, ny;              // grid of tiles (set by the launcher)
 };
 int launch_gemm(const GemmParams& p, hipStream_t s);
+int launch_gemm_ternary(const GemmParams& p, hipStream_t s);
 
-// The GEMM's input planes from fp32 rows: v = x (no norm), or x / rms(x) * norm_w (RMSNorm,
-// model/fastref.py:143-144), or a PrismML rotation of that (signs != null: per block of B
-// columns v' = scale * H (signs * v), H the +-1 Sylvester matrix); xh = fp16(v / xs), xl =
-// fp16(v / xs - xh), with xs[r] the power of two that brings row r below 2^14 (1 for most rows:
-// fp16 holds values up to 65504, and a row past that would give inf and NaN products).
+// The ternary GEMM's digit planes of R rows of K floats (norm_w: times the gain, not yet divided by
+// rms(x)), 4 R K bytes at xp (16-byte aligned). turned: the trit5 rows' column order.
+struct PlanesParams {
+  const float* x;
+  int ldx, K, R;
+  const float* norm_w;
+  int turned;
+  uint8_t* xp;
+};
+int launch_planes(const PlanesParams& p, hipStream_t s);
+
+// The Q8 GEMM's input planes from fp32 rows: v = x (no norm), or x / rms(x) * norm_w (RMSNorm,
+// model/fastref.py:143-144); xh = fp16(v / xs), xl = fp16(v / xs - xh), with xs[r] the power of two
+// that brings row r below 2^14 (1 for most rows: fp16 holds values up to 65504, and a row past that
+// would give inf and NaN products).
 struct PrepParams {
   const float* x;
   int ldx, K, R;
   const float* norm_w;
   float eps;
-  const float* signs;      // rotation, or null
-  int B;
-  float scale;
   _Float16* xh;            // [R][K]
   _Float16* xl;
   float* xs;               // [R]
-  float* rs;               // [R] a rotated input's 1/rms per row (null without a rotation)
 };
 int launch_prep(const PrepParams& p, hipStream_t s);
+
+// A PrismML rotation of R rows: out = scale * H (signs * v) per block of B columns (H the +-1
+// Sylvester matrix), v = x, or x / rms(x) * norm_w with norm_w != null. out: [R][K].
+struct RotateRowsParams {
+  const float* x;
+  int ldx, K, R;
+  const float* norm_w;
+  float eps;
+  const float* signs;
+  int B;
+  float scale;
+  float* rs;               // [R] 1/rms per row (written first)
+  float* out;
+};
+int launch_rotate_rows(const RotateRowsParams& p, hipStream_t s);
 
 // Per position and head: q and k RMS-normalised (their gains), NEOX RoPE on the first rope_n
 // dims at position p0 + r (Q14 table row or theta^(-2i/n)), q scaled by 1/sqrt(hd) into q_out;

@@ -1,9 +1,7 @@
 // Batched prefill kernels: R prompt positions per forward, one weight pass for all of them.
 //
-// The projections run on the matrix cores (v_mfma_f32_32x32x16_f16): four waves of a block decode
-// 256 stored ternary rows into LDS as fp16 weights, 64 columns at a time, while its other four
-// multiply 128 (or 64) positions by the previous 64 columns, x split into two fp16 planes (hi,
-// lo) so the fp32 accumulation sees x to ~22 bits.
+// The ternary projections run on the matrix cores from fp6 digit planes (trx_gemm.hip); the Q8 ones
+// (the DeltaNet beta|alpha rows) here, from fp16 hi and lo planes.
 // Attention, the RoPE/KV append and the Gated DeltaNet recurrence are the one-position rules of
 // the decode kernels applied to every position of the chunk (the recurrence in order).
 
@@ -42,23 +40,20 @@ __device__ __forceinline__ int gm_wrow(int epi, int i, int M) {
   return blockIdx.x * kGmBM + i;
 }
 
-template <int KIND>
 struct GmRaw {
-  uint4 c[KIND == TRX_KIND_Q8 ? 4 : 1];
+  uint4 c[4];
   uint32_t sc;
 };
 
 // NA: position tiles of 32 per wave (2: 128 positions per block; 1: 64, for grids that would
 // otherwise leave part of a round of blocks idle).
-template <int KIND, int EPI, int NA>
-__global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
+template <int EPI, int NA>
+__global__ __launch_bounds__(kGmThreads, 1) void gemm_q8_kernel(GemmParams p) {
   constexpr int BR = 64 * NA;
   // Two buffers of each: a step (64 columns, half a group) is staged into one while the matrix
   // cores read the other.
   __shared__ __align__(16) _Float16 ws[2][kGmBM * kGmLd];
   __shared__ __align__(16) _Float16 xs[2][2][BR * kGmLd];
-  __shared__ uint32_t tsel[16];
-  __shared__ uint2 tsel27[32];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const bool cw = w < 4;                    // a wave that runs the MFMAs
   const int stid = max(tid - kGmStage, 0);  // staging thread index
@@ -66,23 +61,6 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   // K in gridDim.z parts (more than one only for a plain store into p.part): this block's groups
   // g0 .. g0 + G - 1.
   const int G = p.K / kGroup / (int)gridDim.z, g0 = (int)blockIdx.z * G;
-
-  // Weights are decoded by v_perm_b32 from a register pair holding -s, 0, s and 2s as fp16 (s the
-  // group's scale): selector half g(c) = 0x0100 + c * 0x0202 picks (c - 1) * s for code c. trit5:
-  // a code byte b = lo + 9 hi, tsel[lo] = g(d0) | g(d1) << 16 and tsel27[hi] = {g(d2) | g(d3) <<
-  // 16, g(d4)} (hi <= 28 for any byte). 2-bit: tsel[nibble] = g(c0) | g(c1) << 16. No table has
-  // more entries than the LDS has banks, so its reads never conflict (a 256-entry table of the
-  // decoded bytes stalled the LDS a third of the time).
-  if (!cw && stid < 32) {
-    auto gsel = [](int c) { return 0x0100u + 0x0202u * (uint32_t)c; };
-    const int t = stid;
-    if (KIND == TRX_KIND_TERNARY5) {
-      if (t < 9) tsel[t] = gsel(t % 3) | gsel(t / 3) << 16;
-      tsel27[t] = make_uint2(gsel(t % 3) | gsel(t / 3 % 3) << 16, gsel(t / 9 % 3));
-    } else if (KIND == TRX_KIND_TERNARY) {
-      if (t < 16) tsel[t] = gsel(t & 3) | gsel(t >> 2) << 16;
-    }
-  }
 
   // Staging roles (waves 4-7): staging thread t decodes the 128 codes of LDS row t (two halves
   // of 64), and copies eight 16-byte pieces of the two x planes.
@@ -94,27 +72,15 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   const __amdgpu_buffer_rsrc_t rxh = make_rsrc(p.xh, (uint32_t)((size_t)p.R * p.K * 2));
   const __amdgpu_buffer_rsrc_t rxl = make_rsrc(p.xl, (uint32_t)((size_t)p.R * p.K * 2));
 
-  auto load_w = [&](GmRaw<KIND>& raw, int g, int shalf) {
-    if (KIND == TRX_KIND_TERNARY5) {
-      const uint32_t o = (uint32_t)p.code_off + 26u * (uint32_t)g + (shalf ? 12u : 0u);
-      const auto a = __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + (o & ~3u), 0, 0);
-      raw.c[0] = make_uint4(a[0], a[1], a[2], a[3]);
-      raw.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
-    } else if (KIND == TRX_KIND_TERNARY) {
-      const uint32_t o = (uint32_t)p.code_off + 32u * (uint32_t)g + 16u * (uint32_t)shalf;
-      const auto a = __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + o, 0, 0);
-      raw.c[0] = make_uint4(a[0], a[1], a[2], a[3]);
-      raw.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
-    } else {
-      const uint32_t o = (uint32_t)p.code_off + 128u * (uint32_t)g + 64u * (uint32_t)shalf;
+  auto load_w = [&](GmRaw& raw, int g, int shalf) {
+    const uint32_t o = (uint32_t)p.code_off + 128u * (uint32_t)g + 64u * (uint32_t)shalf;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const auto a = __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + o + 16u * k, 0, 0);
-        raw.c[k] = make_uint4(a[0], a[1], a[2], a[3]);
-      }
-      // The two 32-column group scales of this half (groups 4g + 2 shalf and the next).
-      raw.sc = __builtin_amdgcn_raw_buffer_load_b32(rw, rbase + 2u * (4u * (uint32_t)g + 2u * (uint32_t)shalf), 0, 0);
+    for (int k = 0; k < 4; ++k) {
+      const auto a = __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + o + 16u * k, 0, 0);
+      raw.c[k] = make_uint4(a[0], a[1], a[2], a[3]);
     }
+    // The two 32-column group scales of this half (groups 4g + 2 shalf and the next).
+    raw.sc = __builtin_amdgcn_raw_buffer_load_b32(rw, rbase + 2u * (4u * (uint32_t)g + 2u * (uint32_t)shalf), 0, 0);
   };
   constexpr int XQ = BR * 8 / kGmStage;            // 16-byte x pieces per thread, plane and step
   // x of step st (columns 64 st .. + 63): thread t moves pieces t + 256 q (row piece / 8, 8 columns).
@@ -132,91 +98,21 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   // Decoded weights of this thread's 64 codes: 32 dwords of fp16 pairs, times the scale (0 for
   // a row past M, whose codes were read from row 0). The half of the group (shc, a compile-time
   // constant) is also the LDS buffer. No branch: one block of code per half.
-  auto stage_w = [&](const GmRaw<KIND>& raw, int g, auto shc) {
-    constexpr int shalf = decltype(shc)::value, buf = shalf;
+  auto stage_w = [&](const GmRaw& raw, auto shc) {
+    constexpr int buf = decltype(shc)::value;
     uint32_t D[32];
     const uint32_t sc = wvalid ? raw.sc : 0u;
-    if (KIND == TRX_KIND_Q8) {
-      // int8 -> fp16 exactly, times the 32-column group's scale in fp16 (fp16(q * s)).
-      const uint32_t dw[16] = {raw.c[0].x, raw.c[0].y, raw.c[0].z, raw.c[0].w, raw.c[1].x, raw.c[1].y,
-                               raw.c[1].z, raw.c[1].w, raw.c[2].x, raw.c[2].y, raw.c[2].z, raw.c[2].w,
-                               raw.c[3].x, raw.c[3].y, raw.c[3].z, raw.c[3].w};
-      const uint32_t s0 = sc & 0xFFFFu, s1 = sc >> 16;
+    // int8 -> fp16 exactly, times the 32-column group's scale in fp16 (fp16(q * s)).
+    const uint32_t dw[16] = {raw.c[0].x, raw.c[0].y, raw.c[0].z, raw.c[0].w, raw.c[1].x, raw.c[1].y,
+                             raw.c[1].z, raw.c[1].w, raw.c[2].x, raw.c[2].y, raw.c[2].z, raw.c[2].w,
+                             raw.c[3].x, raw.c[3].y, raw.c[3].z, raw.c[3].w};
+    const uint32_t s0 = sc & 0xFFFFu, s1 = sc >> 16;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        auto q = [&](int b) { return half_bits((float)(int8_t)(uint8_t)(dw[j] >> (8 * b))); };
-        const uint32_t s2 = j < 8 ? (s0 | s0 << 16) : (s1 | s1 << 16);
-        D[2 * j] = pk_mul_h2(q(0) | q(1) << 16, s2);
-        D[2 * j + 1] = pk_mul_h2(q(2) | q(3) << 16, s2);
-      }
-    } else {
-      // The permute pair: bytes 0-3 {-s, 0}, bytes 4-7 {s, 2s} (fp16(1 * s), fp16(2 * s)).
-      const uint32_t s16 = sc & 0xFFFFu;
-      const uint32_t plo = s16 ^ 0x8000u, phi = pk_mul_h2(s16 | s16 << 16, 0x40003C00u);
-      auto wp = [&](uint32_t sel) { return __builtin_amdgcn_perm(phi, plo, sel); };
-      if (KIND == TRX_KIND_TERNARY5) {
-        const uint32_t o = (uint32_t)p.code_off + 26u * (uint32_t)g + (shalf ? 12u : 0u);
-        const uint32_t sh = o & 3u;
-        const uint32_t d0 = __builtin_amdgcn_alignbyte(raw.c[0].y, raw.c[0].x, sh);
-        const uint32_t d1 = __builtin_amdgcn_alignbyte(raw.c[0].z, raw.c[0].y, sh);
-        const uint32_t d2 = __builtin_amdgcn_alignbyte(raw.c[0].w, raw.c[0].z, sh);
-        const uint32_t d3 = __builtin_amdgcn_alignbyte(0u, raw.c[0].w, sh);
-        const uint32_t dw[4] = {d0, d1, d2, d3};
-        // Byte j's selectors: lo pair (d0, d1) and hi {(d2, d3), d4}.
-        auto sel = [&](int j, uint32_t& lo, uint2& hi) {
-          const uint32_t b = (dw[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-          const uint32_t h = (b * 57u) >> 9;          // b / 9 for every byte value
-          lo = tsel[b - 9u * h];
-          hi = tsel27[h];
-        };
-        // An even byte's five codes start a dword, the odd byte's five follow: five dwords.
-        auto pair5 = [&](int j, uint32_t* out) {
-          uint32_t e9, o9;
-          uint2 e27, o27;
-          sel(j, e9, e27);
-          sel(j + 1, o9, o27);
-          out[0] = wp(e9);
-          out[1] = wp(e27.x);
-          out[2] = wp(e27.y | o9 << 16);
-          out[3] = wp(__builtin_amdgcn_alignbit(o27.x, o9, 16));
-          out[4] = wp(__builtin_amdgcn_alignbit(o27.y, o27.x, 16));
-        };
-        if constexpr (shalf == 0) {
-          // bytes 0..12: codes 0..64, of which 0..63 are this half's
-#pragma unroll
-          for (int i = 0; i < 6; ++i) pair5(2 * i, D + 5 * i);
-          uint32_t e9;
-          uint2 e27;
-          sel(12, e9, e27);
-          D[30] = wp(e9);
-          D[31] = wp(e27.x);
-        } else {
-          // bytes 12..25: codes 60..129; this half takes 64..127
-          uint32_t e9, o9;
-          uint2 e27, o27;
-          sel(0, e9, e27);
-          sel(1, o9, o27);
-          D[0] = wp(e27.y | o9 << 16);
-          D[1] = wp(__builtin_amdgcn_alignbit(o27.x, o9, 16));
-          D[2] = wp(__builtin_amdgcn_alignbit(o27.y, o27.x, 16));
-#pragma unroll
-          for (int i = 1; i < 6; ++i) pair5(2 * i, D + 5 * i - 2);
-          uint32_t t[5];
-          pair5(12, t);
-          D[28] = t[0];
-          D[29] = t[1];
-          D[30] = t[2];
-          D[31] = t[3];
-        }
-      } else {
-        const uint32_t dw[4] = {raw.c[0].x, raw.c[0].y, raw.c[0].z, raw.c[0].w};
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const uint32_t b = (dw[j >> 2] >> (8 * (j & 3))) & 0xFFu;
-          D[2 * j] = wp(tsel[b & 15u]);
-          D[2 * j + 1] = wp(tsel[b >> 4]);
-        }
-      }
+    for (int j = 0; j < 16; ++j) {
+      auto q = [&](int b) { return half_bits((float)(int8_t)(uint8_t)(dw[j] >> (8 * b))); };
+      const uint32_t s2 = j < 8 ? (s0 | s0 << 16) : (s1 | s1 << 16);
+      D[2 * j] = pk_mul_h2(q(0) | q(1) << 16, s2);
+      D[2 * j + 1] = pk_mul_h2(q(2) | q(3) << 16, s2);
     }
     uint4* dst = (uint4*)(ws[buf] + srow * kGmLd);
 #pragma unroll
@@ -247,7 +143,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   // steps of latency cover). The loop is unrolled by two, so a step's registers and buffers are
   // fixed per half.
   const int NS = 2 * G;
-  GmRaw<KIND> raw[2];
+  GmRaw raw[2];
   uint4 xr[2][2 * XQ];
   auto load_step = [&](int st, int slot) {
     load_w(raw[slot], g0 + (st >> 1), st & 1);
@@ -255,7 +151,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   };
   // A step's half is its register slot and LDS buffer: st & 1 == slot.
   auto stage_step = [&](int st, auto slot) {
-    stage_w(raw[decltype(slot)::value], g0 + (st >> 1), slot);
+    stage_w(raw[decltype(slot)::value], slot);
     stage_x(xr[decltype(slot)::value], decltype(slot)::value);
   };
   const std::integral_constant<int, 0> I0;
@@ -292,7 +188,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   if (!cw) {
     load_step(0, 0);
     load_step(1, 1);                      // NS >= 2: K is a multiple of 128
-    __syncthreads();                      // the code tables are written
+    __syncthreads();
     stage_step(0, I0);
     load_step(min(2, NS - 1), 0);
     __syncthreads();
@@ -354,19 +250,19 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(const float* part, int 
   }
 }
 
-template <int KIND, int NA>
-static void gemm_dispatch(const GemmParams& p, dim3 grid, hipStream_t s) {
+template <int NA>
+static void gemm_q8_dispatch(const GemmParams& p, dim3 grid, hipStream_t s) {
   if (p.epi == GM_SWIGLU)
-    hipLaunchKernelGGL((gemm_kernel<KIND, GM_SWIGLU, NA>), grid, dim3(kGmThreads), 0, s, p);
+    hipLaunchKernelGGL((gemm_q8_kernel<GM_SWIGLU, NA>), grid, dim3(kGmThreads), 0, s, p);
   else if (p.epi == GM_RESID)
-    hipLaunchKernelGGL((gemm_kernel<KIND, GM_RESID, NA>), grid, dim3(kGmThreads), 0, s, p);
+    hipLaunchKernelGGL((gemm_q8_kernel<GM_RESID, NA>), grid, dim3(kGmThreads), 0, s, p);
   else
-    hipLaunchKernelGGL((gemm_kernel<KIND, GM_STORE, NA>), grid, dim3(kGmThreads), 0, s, p);
+    hipLaunchKernelGGL((gemm_q8_kernel<GM_STORE, NA>), grid, dim3(kGmThreads), 0, s, p);
 }
 
 int launch_gemm(const GemmParams& p, hipStream_t s) {
-  TRX_CHECK(p.kind == TRX_KIND_TERNARY || p.kind == TRX_KIND_TERNARY5 || p.kind == TRX_KIND_Q8, TRX_E_INVALID,
-            "prefill GEMM: weight kind %d unsupported", p.kind);
+  if (p.kind == TRX_KIND_TERNARY || p.kind == TRX_KIND_TERNARY5) return launch_gemm_ternary(p, s);
+  TRX_CHECK(p.kind == TRX_KIND_Q8, TRX_E_INVALID, "prefill GEMM: weight kind %d unsupported", p.kind);
   TRX_CHECK(p.M >= 1 && p.K >= kGroup && p.K % kGroup == 0 && p.R >= 1, TRX_E_INVALID,
             "prefill GEMM: M=%d K=%d R=%d", p.M, p.K, p.R);
   TRX_CHECK(p.epi != GM_SWIGLU || p.M % 2 == 0, TRX_E_INVALID, "prefill GEMM: SwiGLU needs an even M");
@@ -392,16 +288,8 @@ int launch_gemm(const GemmParams& p, hipStream_t s) {
         break;
       }
   const dim3 grid(nx, cdiv(p.R, small ? 64 : 128), kp);
-  if (p.kind == TRX_KIND_TERNARY5) {
-    if (small) gemm_dispatch<TRX_KIND_TERNARY5, 1>(p, grid, s);
-    else gemm_dispatch<TRX_KIND_TERNARY5, 2>(p, grid, s);
-  } else if (p.kind == TRX_KIND_TERNARY) {
-    if (small) gemm_dispatch<TRX_KIND_TERNARY, 1>(p, grid, s);
-    else gemm_dispatch<TRX_KIND_TERNARY, 2>(p, grid, s);
-  } else {
-    if (small) gemm_dispatch<TRX_KIND_Q8, 1>(p, grid, s);
-    else gemm_dispatch<TRX_KIND_Q8, 2>(p, grid, s);
-  }
+  if (small) gemm_q8_dispatch<1>(p, grid, s);
+  else gemm_q8_dispatch<2>(p, grid, s);
   TRX_LAUNCHED();
   if (kp > 1) {
     hipLaunchKernelGGL(gemm_parts_kernel, dim3(p.R), dim3(256), 0, s, p.part, kp, p.R, p.M, p.ldy, p.y);
@@ -511,42 +399,26 @@ __global__ __launch_bounds__(256) void prep_vec_kernel(PrepParams p) {
   }
 }
 
-// Rotated input: one block of B threads per (rotation block, position), as rotate_kernel does for
-// one vector (the whole row's sum of squares, the butterflies by shuffles then LDS).
-// The rotated input's row statistics, one block of 256 threads per position: the RMSNorm scale
-// 1/rms(x) (1 without a norm) and the power of two that keeps the row's planes finite. Every
-// output of a rotation block is bounded by scale * B times the row's largest |x * gain| (times
-// 1/rms), which sets one scale for all of the row's blocks.
-__global__ __launch_bounds__(256) void prep_rot_stats_kernel(PrepParams p) {
+// A rotated input's 1/rms per row (1 without a norm), one block of 256 threads per position.
+__global__ __launch_bounds__(256) void rotate_stats_kernel(RotateRowsParams p) {
   __shared__ float red[16];
   const int r = blockIdx.x, t = threadIdx.x;
   const float* x = p.x + (size_t)r * p.ldx;
-  float ss = 0.f, am = 0.f;
-  for (int i = t; i < p.K; i += 256) {
-    ss += x[i] * x[i];
-    am = fmaxf(am, fabsf(p.norm_w ? x[i] * p.norm_w[i] : x[i]));
-  }
+  float ss = 0.f;
+  for (int i = t; i < p.K; i += 256) ss += x[i] * x[i];
   const float tot = block_sum(ss, red);
-  const float amax = block_max(am, red);
-  const float rsn = p.norm_w ? 1.0f / sqrtf(tot / (float)p.K + p.eps) : 1.f;
-  float down, up;
-  row_scale(fabsf(p.scale) * (float)p.B * amax * rsn, down, up);
-  if (t == 0) {
-    p.xs[r] = up;
-    p.rs[r] = rsn;
-  }
+  if (t == 0) p.rs[r] = 1.0f / sqrtf(tot / (float)p.K + p.eps);
 }
 
 // Rotated input: one block of B threads per (rotation block, position), as rotate_kernel does for
-// one vector (the butterflies by shuffles then LDS), with the row's statistics from above.
-__global__ __launch_bounds__(1024) void prep_rot_kernel(PrepParams p) {
+// one vector (the butterflies by shuffles then LDS).
+__global__ __launch_bounds__(1024) void rotate_rows_kernel(RotateRowsParams p) {
   __shared__ float v[1024];
   const int t = threadIdx.x, B = blockDim.x, c = blockIdx.x * B + t, r = blockIdx.y;
   const int lane = t & 63;
   const float* x = p.x + (size_t)r * p.ldx;
   float a = x[c] * p.signs[c];
   if (p.norm_w) a *= p.norm_w[c] * p.rs[r];
-  const float down = 1.0f / p.xs[r];               // a power of two: exact
   for (int h = 1; h < 64; h <<= 1) {
     const float o = __shfl_xor(a, h, 64);
     a = (lane & h) ? o - a : a + o;
@@ -558,22 +430,29 @@ __global__ __launch_bounds__(1024) void prep_rot_kernel(PrepParams p) {
     __syncthreads();
     a = (t & h) ? o - a : a + o;
   }
-  store_hilo(p, (size_t)r * p.K + c, a * p.scale * down);
+  p.out[(size_t)r * p.K + c] = a * p.scale;
+}
+
+int launch_rotate_rows(const RotateRowsParams& p, hipStream_t s) {
+  TRX_CHECK(p.R >= 1 && p.K >= 1 && p.ldx >= p.K && p.rs && p.out, TRX_E_INVALID, "prefill rotation: R=%d K=%d", p.R,
+            p.K);
+  TRX_CHECK(p.B >= 64 && p.B <= 1024 && (p.B & (p.B - 1)) == 0 && p.K % p.B == 0, TRX_E_INVALID,
+            "prefill input: rotation block %d over %d columns unsupported", p.B, p.K);
+  if (p.norm_w) {
+    hipLaunchKernelGGL(rotate_stats_kernel, dim3(p.R), dim3(256), 0, s, p);
+    TRX_LAUNCHED();
+  }
+  hipLaunchKernelGGL(rotate_rows_kernel, dim3(p.K / p.B, p.R), dim3(p.B), 0, s, p);
+  TRX_LAUNCHED();
+  return TRX_OK;
 }
 
 int launch_prep(const PrepParams& p, hipStream_t s) {
   TRX_CHECK(p.R >= 1 && p.K >= 1 && p.ldx >= p.K && p.xs, TRX_E_INVALID, "prefill input: R=%d K=%d", p.R, p.K);
-  if (p.signs) {
-    TRX_CHECK(p.B >= 64 && p.B <= 1024 && (p.B & (p.B - 1)) == 0 && p.K % p.B == 0, TRX_E_INVALID,
-              "prefill input: rotation block %d over %d columns unsupported", p.B, p.K);
-    TRX_CHECK(p.rs, TRX_E_INVALID, "prefill input: a rotation needs the row-scale buffer");
-    hipLaunchKernelGGL(prep_rot_stats_kernel, dim3(p.R), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(prep_rot_kernel, dim3(p.K / p.B, p.R), dim3(p.B), 0, s, p);
-  } else if (p.K % 4 == 0 && p.ldx % 4 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.norm_w & 15) == 0) {
+  if (p.K % 4 == 0 && p.ldx % 4 == 0 && ((uintptr_t)p.x & 15) == 0 && ((uintptr_t)p.norm_w & 15) == 0)
     hipLaunchKernelGGL(prep_vec_kernel, dim3(p.R), dim3(256), 0, s, p);
-  } else {
+  else
     hipLaunchKernelGGL(prep_kernel, dim3(p.R), dim3(256), 0, s, p);
-  }
   TRX_LAUNCHED();
   return TRX_OK;
 }
@@ -1184,21 +1063,6 @@ TRX_API int trx_gemm_ternary_f32(const uint8_t* rows, int kind, int M, int K, co
   TRX_CHECK(K >= kGroup && K % kGroup == 0 && M >= 1, TRX_E_INVALID, "trx_gemm_ternary_f32: M=%d K=%d", M, K);
   const int row_bytes = kind == TRX_KIND_Q8 ? kBeat * cdiv(K / 32, 16) + K : row_geom(kind, K).row_bytes;
   const int code_off = kind == TRX_KIND_Q8 ? kBeat * cdiv(K / 32, 16) : row_geom(kind, K).code_off;
-  _Float16* xh = (_Float16*)workspace;
-  _Float16* xl = xh + (size_t)n * K;
-  float* xs = (float*)(xl + (size_t)n * K);
-  PrepParams pp = {};
-  pp.x = x;
-  pp.ldx = K;
-  pp.K = K;
-  pp.R = n;
-  pp.norm_w = norm_w;
-  pp.eps = eps;
-  pp.xh = xh;
-  pp.xl = xl;
-  pp.xs = xs;
-  int rc;
-  if ((rc = launch_prep(pp, (hipStream_t)s))) return rc;
   GemmParams g = {};
   g.W = rows;
   g.w_bytes = (uint32_t)std::min<size_t>((size_t)M * row_bytes + 16, 0xFFFFFFF0u);
@@ -1207,10 +1071,37 @@ TRX_API int trx_gemm_ternary_f32(const uint8_t* rows, int kind, int M, int K, co
   g.K = K;
   g.row_bytes = row_bytes;
   g.code_off = code_off;
-  g.xh = xh;
-  g.xl = xl;
-  g.xs = xs;
   g.R = n;
+  int rc;
+  if (kind == TRX_KIND_Q8) {
+    PrepParams pp = {};
+    pp.x = x;
+    pp.ldx = K;
+    pp.K = K;
+    pp.R = n;
+    pp.norm_w = norm_w;
+    pp.eps = eps;
+    pp.xh = (_Float16*)workspace;
+    pp.xl = pp.xh + (size_t)n * K;
+    pp.xs = (float*)(pp.xl + (size_t)n * K);
+    if ((rc = launch_prep(pp, (hipStream_t)s))) return rc;
+    g.xh = pp.xh;
+    g.xl = pp.xl;
+    g.xs = pp.xs;
+  } else {
+    PlanesParams pp = {};
+    pp.x = x;
+    pp.ldx = K;
+    pp.K = K;
+    pp.R = n;
+    pp.norm_w = norm_w;
+    pp.turned = kind == TRX_KIND_TERNARY5;
+    pp.xp = (uint8_t*)workspace;
+    if ((rc = launch_planes(pp, (hipStream_t)s))) return rc;
+    g.xp = pp.xp;
+    g.norm = norm_w != nullptr;
+    g.eps = eps;
+  }
   g.epi = epilogue == TRX_EPI_STORE ? GM_STORE : epilogue == TRX_EPI_RESID ? GM_RESID : GM_SWIGLU;
   g.y = y;
   g.ldy = epilogue == TRX_EPI_SWIGLU ? M / 2 : M;
