@@ -173,6 +173,20 @@ struct ScoreParams {
   float* nll;
 };
 int launch_score(const ScoreParams& p, hipStream_t s);
+// The same for R positions at once: the normed hidden states of residual rows x [R][n] into hid, and
+// with logits [R][vocab] nll[r] = logsumexp(logits[r]) - logits[r][target[r]].
+struct ScoreRowsParams {
+  const float* x;
+  const float* out_norm;
+  float eps;
+  int n, R;
+  float* hid;
+  const float* logits;
+  int vocab;
+  const int* target;
+  float* nll;
+};
+int launch_score_rows(const ScoreRowsParams& p, hipStream_t s);
 
 int launch_embed(const EmbedParams& p, hipStream_t s);
 // Prefill: the embeddings of the tokens fed at positions p0 .. p0 + R - 1 into X [R][n_embd]

@@ -672,6 +672,65 @@ int launch_score(const ScoreParams& p, hipStream_t s) {
   return TRX_OK;
 }
 
+__global__ __launch_bounds__(256) void hidden_rows_kernel(ScoreRowsParams p) {
+  __shared__ float red[16];
+  const float* x = p.x + (size_t)blockIdx.x * p.n;
+  float ss = 0.f;
+  for (int i = threadIdx.x; i < p.n; i += 256) ss += x[i] * x[i];
+  const float r = 1.0f / sqrtf(block_sum(ss, red) / (float)p.n + p.eps);
+  for (int i = threadIdx.x; i < p.n; i += 256) p.hid[(size_t)blockIdx.x * p.n + i] = x[i] * r * p.out_norm[i];
+}
+
+// One block per position, one pass over its logits: each thread keeps a running maximum of its
+// columns and the sum of exponentials under it, the block combines them. Bound by reading the logits
+// the head's GEMM has just written.
+__global__ __launch_bounds__(1024) void nll_rows_kernel(ScoreRowsParams p) {
+  __shared__ float rm[16], rs[16];
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const float* lg = p.logits + (size_t)r * p.vocab;
+  constexpr int U = 8;
+  float m = -INFINITY, s = 0.f;
+  for (int i0 = tid; i0 < p.vocab; i0 += 1024 * U) {
+    float v[U], top = m;
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      v[k] = i0 + 1024 * k < p.vocab ? lg[i0 + 1024 * k] : -INFINITY;
+      top = fmaxf(top, v[k]);
+    }
+    if (top == -INFINITY) continue;
+    s *= expf(m - top);
+#pragma unroll
+    for (int k = 0; k < U; ++k) s += expf(v[k] - top);
+    m = top;
+  }
+  const float wm = wave_max(m);
+  s = wave_sum(m == -INFINITY ? 0.f : s * expf(m - wm));
+  if (lane == 0) {
+    rm[tid >> 6] = wm;
+    rs[tid >> 6] = s;
+  }
+  __syncthreads();
+  if (tid) return;
+  float bm = rm[0], t = 0.f;
+  for (int i = 1; i < 16; ++i) bm = fmaxf(bm, rm[i]);
+  for (int i = 0; i < 16; ++i) t += rm[i] == -INFINITY ? 0.f : rs[i] * expf(rm[i] - bm);
+  p.nll[r] = (bm + logf(t)) - lg[p.target[r]];
+}
+
+int launch_score_rows(const ScoreRowsParams& p, hipStream_t s) {
+  TRX_CHECK(p.R >= 1 && p.n > 0 && (!p.hid || (p.x && p.out_norm)) && (!p.logits || (p.nll && p.target)), TRX_E_INVALID,
+            "score: bad arguments");
+  if (p.hid) {
+    hipLaunchKernelGGL(hidden_rows_kernel, dim3(p.R), dim3(256), 0, s, p);
+    TRX_LAUNCHED();
+  }
+  if (p.logits) {
+    hipLaunchKernelGGL(nll_rows_kernel, dim3(p.R), dim3(1024), 0, s, p);
+    TRX_LAUNCHED();
+  }
+  return TRX_OK;
+}
+
 int launch_finalize(const int* pos, const int* n_prompt, unsigned long long* slot, int* out, int max_out,
                     hipStream_t s) {
   hipLaunchKernelGGL(finalize_kernel, dim3(1), dim3(64), 0, s, pos, n_prompt, slot, out, max_out);

@@ -408,7 +408,7 @@ class Decoder:
         """(nll [T-1] of tokens[1:] given their prefix, final normed hidden states [T, n_embd]),
         teacher-forced from position 0 after a reset (HybridRef.score, model/fastref.py:263-273).
         The log-sum-exp over the vocabulary runs on the GPU in float32; `chunk` is accepted for
-        the reference's signature (the GPU scores one position at a time)."""
+        the reference's signature (the library chooses its own blocks)."""
         t = np.ascontiguousarray(np.asarray(tokens, dtype=np.int32).reshape(-1))
         if t.size == 0:
             raise ValueError("no tokens to score")
