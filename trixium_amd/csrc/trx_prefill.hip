@@ -927,76 +927,110 @@ __global__ void dn_conv_tail_kernel(DnRowsParams p) {
   for (int i = 0; i < p.Kc - 1; ++i) p.conv_state[(size_t)i * p.C + c] = keep[i];
 }
 
-// The recurrence of one value head over the chunk, one pass of state rows per block (8 rows at
-// HK = 128, 16 at 64; 256 threads): a row's HK columns over HK/4 lanes (a float4 each), row sums by
-// DPP. First every block computes its head's decay and beta gates of all the chunk's positions at
-// once (into LDS), so the serial loop carries only the state's arithmetic; each position's k, q
-// and v are loaded kScanAhead positions ahead. The per-position arithmetic is
-// dn_recur_fixed_kernel's.
-constexpr int kScanAhead = 4;          // positions whose inputs are in flight ahead of the scan
+// The recurrence of one value head over the chunk: 16 state rows per block of 256 threads, a row's HK
+// columns over 16 lanes, row sums by DPP. First every block computes its head's decay and beta gates
+// of all the chunk's positions at once (into LDS), so the serial loop carries only the state's
+// arithmetic; k, q and v come through LDS, kScanTile positions at a time, the next tile's loads in
+// flight meanwhile. The per-position arithmetic is dn_recur_fixed_kernel's.
+// Bound by vector issue: the 6144 rows of the 27B shape are 1536 waves of ~50 operations a position.
+// With 32 lanes a row (8 rows a block, two lane swaps a position through LDS, k and q loaded by every
+// wave) a 1024-position chunk took 558 us; 212 us this way.
+constexpr int kScanTile = 16;
 constexpr int kScanRMax = 8192;        // chunk positions whose gates fit the LDS (64 KB)
-template <int HK>
-constexpr int scan_rows() { return 4 * (64 / (HK / 4)); }
-// Sum over a row's LPR lanes (16 or 32, aligned), every lane getting it: DPP within each 16-lane
-// row, then one lane swap between the two rows of a 32-lane row.
-template <int LPR>
-__device__ __forceinline__ float row_sum(float v) {
-  static_assert(LPR == 16 || LPR == 32, "row width");
-  v = row16_sum(v);
-  if (LPR == 32) v += __shfl_xor(v, 16, 64);
-  return v;
-}
+constexpr int kScanRows = 16;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 template <int HK>
 __global__ __launch_bounds__(256) void dn_scan_kernel(DnRowsParams p) {
-  constexpr int LPR = HK / 4, RPW = 64 / LPR, RB = scan_rows<HK>();
-  extern __shared__ float gates[];      // [R] decay, then [R] beta
-  const int h = blockIdx.x, rb = blockIdx.y, t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int sub = lane / LPR, c4 = lane % LPR;
+  constexpr int V = HK / 64;            // float4s of a row per lane: columns 4 c + 64 i
+  extern __shared__ float2 gates[];     // decay and beta of whole tiles' positions
+  __shared__ __align__(16) float kq[2][kScanTile][2 * HK];
+  __shared__ float vs[2][kScanTile][kScanRows];
+  const int h = blockIdx.x, rb = blockIdx.y, t = threadIdx.x, c = t & 15, tr = t >> 4;
   const int nk = p.nk, kh = h % nk, hv = p.hv;
-  const int jr = rb * RB + w * RPW + sub;
-  float4* S = (float4*)(p.S + (size_t)h * hv * HK);
-  float4 sv = S[jr * LPR + c4];
+  const int row = rb * kScanRows + tr;
+  const bool live = row < hv;
+  f32x4_t* S = (f32x4_t*)(p.S + ((size_t)h * hv + (live ? row : 0)) * HK) + c;
+  f32x4_t s[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) s[i] = S[16 * i];
   const float Ah = p.A[h], dth = p.dt[h];
-  for (int r = t; r < p.R; r += 256) {
-    const float a = p.ba[(size_t)r * 2 * p.nv + p.nv + h] + dth;
-    const float sp = a > 20.f ? a : log1pf(expf(a));
-    gates[r] = expf(sp * Ah);
-    gates[p.R + r] = sigmoidf_(p.ba[(size_t)r * 2 * p.nv + h]);
+  // Positions past the last leave the state as it is.
+  for (int r = t; r < (p.R + kScanTile - 1) / kScanTile * kScanTile; r += 256) {
+    float2 g = make_float2(1.f, 0.f);
+    if (r < p.R) {
+      const float a = p.ba[(size_t)r * 2 * p.nv + p.nv + h] + dth;
+      const float sp = a > 20.f ? a : log1pf(expf(a));
+      g = make_float2(expf(sp * Ah), sigmoidf_(p.ba[(size_t)r * 2 * p.nv + h]));
+    }
+    gates[r] = g;
   }
-  const float qs = 1.0f / sqrtf((float)HK);
-  auto ld = [&](int r, float4& k4, float4& q4, float& vj) {
-    const float* cr = p.conv_out + (size_t)r * p.C;
-    k4 = *(const float4*)(cr + p.nq + kh * HK + 4 * c4);
-    q4 = *(const float4*)(cr + kh * HK + 4 * c4);
-    vj = cr[2 * p.nq + h * hv + jr];
+  // Thread (tr, c) stages position tr of a tile: its pieces of k and q, and v of the block's row c.
+  f32x4_t kn[V], qn[V];
+  float vn;
+  const int vrow = min(rb * kScanRows + c, hv - 1);
+  auto load = [&](int r0) {
+    const float* cr = p.conv_out + (size_t)min(r0 + tr, p.R - 1) * p.C;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      kn[i] = *(const f32x4_t*)(cr + p.nq + kh * HK + 4 * c + 64 * i);
+      qn[i] = *(const f32x4_t*)(cr + kh * HK + 4 * c + 64 * i);
+    }
+    vn = cr[2 * p.nq + h * hv + vrow];
   };
-  // A ring of the next kScanAhead positions' inputs in registers: a position's loads are issued
-  // kScanAhead positions before it is used, so their latency is covered by that many steps of the
-  // recurrence (one step is shorter than a memory round trip).
-  float4 k4[kScanAhead], q4[kScanAhead];
-  float vj[kScanAhead];
+  auto store = [&](int buf) {
 #pragma unroll
-  for (int u = 0; u < kScanAhead; ++u)
-    if (u < p.R) ld(u, k4[u], q4[u], vj[u]);
+    for (int i = 0; i < V; ++i) {
+      *(f32x4_t*)&kq[buf][tr][4 * c + 64 * i] = kn[i];
+      *(f32x4_t*)&kq[buf][tr][HK + 4 * c + 64 * i] = qn[i];
+    }
+    vs[buf][tr][c] = vn;
+  };
+  const float qs = 1.0f / sqrtf((float)HK);
+  float* o = p.o_raw + (size_t)h * hv + row;
+  load(0);
+  store(0);
+  load(kScanTile);
   __syncthreads();
-  for (int r0 = 0; r0 < p.R; r0 += kScanAhead)
+  for (int r0 = 0, buf = 0; r0 < p.R; r0 += kScanTile, buf ^= 1) {
+    float keep = 0.f;
 #pragma unroll
-  for (int u = 0; u < kScanAhead; ++u) {
-    const int r = r0 + u;
-    if (r >= p.R) break;
-    const float4 ck = k4[u], cq = q4[u];
-    const float cv = vj[u];
-    if (r + kScanAhead < p.R) ld(r + kScanAhead, k4[u], q4[u], vj[u]);
-    const float decay = gates[r], beta = gates[p.R + r];
-    float4 s4 = make_float4(sv.x * decay, sv.y * decay, sv.z * decay, sv.w * decay);
-    const float dot = row_sum<LPR>((s4.x * ck.x + s4.y * ck.y) + (s4.z * ck.z + s4.w * ck.w));
-    const float delta = (cv - dot) * beta;
-    s4 = make_float4(s4.x + delta * ck.x, s4.y + delta * ck.y, s4.z + delta * ck.z, s4.w + delta * ck.w);
-    sv = s4;
-    const float oq = row_sum<LPR>((s4.x * cq.x + s4.y * cq.y) + (s4.z * cq.z + s4.w * cq.w));
-    if (c4 == 0) p.o_raw[(size_t)r * p.nv * hv + (size_t)h * hv + jr] = oq * qs;
+    for (int u = 0; u < kScanTile; ++u) {
+      const float2 g = gates[r0 + u];
+      const float decay = g.x, beta = g.y, vj = vs[buf][u][tr];
+      f32x4_t k[V], q[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        k[i] = *(const f32x4_t*)&kq[buf][u][4 * c + 64 * i];
+        q[i] = *(const f32x4_t*)&kq[buf][u][HK + 4 * c + 64 * i];
+      }
+      // Two chains of multiply-adds per sum.
+      float d0 = 0.f, d1 = 0.f, q0 = 0.f, q1 = 0.f;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        s[i] = s[i] * decay;
+        d0 = fmaf(s[i].y, k[i].y, fmaf(s[i].x, k[i].x, d0));
+        d1 = fmaf(s[i].w, k[i].w, fmaf(s[i].z, k[i].z, d1));
+      }
+      const float delta = (vj - row16_sum(d0 + d1)) * beta;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        s[i] = s[i] + delta * k[i];
+        q0 = fmaf(s[i].y, q[i].y, fmaf(s[i].x, q[i].x, q0));
+        q1 = fmaf(s[i].w, q[i].w, fmaf(s[i].z, q[i].z, q1));
+      }
+      const float oq = row16_sum(q0 + q1);
+      keep = c == u ? oq : keep;                       // lane c keeps position c of the tile
+    }
+    if (live && r0 + c < p.R) o[(size_t)(r0 + c) * p.nv * hv] = keep * qs;
+    // The buffer that the last tile left is read by nobody past the last barrier.
+    store(buf ^ 1);
+    load(r0 + 2 * kScanTile);
+    __syncthreads();
   }
-  S[jr * LPR + c4] = sv;
+  if (live) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) S[16 * i] = s[i];
+  }
 }
 
 // Gated RMSNorm of every (position, value head), into the grouped output order.
@@ -1015,7 +1049,7 @@ __global__ void dn_gnorm_rows_kernel(DnRowsParams p) {
 }
 
 int launch_dn_rows(const DnRowsParams& p, hipStream_t s) {
-  const int rb = p.hk == 128 ? scan_rows<128>() : scan_rows<64>();
+  const int rb = p.hk == 128 ? 8 : 16;
   TRX_CHECK(p.R >= 1 && p.R <= kScanRMax && p.hk <= 256 && p.C % p.hk == 0 && p.Kc >= 1 && p.Kc <= 9 &&
             p.nv % p.nk == 0 && (p.hk == 64 || p.hk == 128) && p.hv % rb == 0 && p.hv <= 1024, TRX_E_INVALID,
             "prefill DeltaNet: unsupported geometry hk=%d hv=%d Kc=%d (chunk %d)", p.hk, p.hv, p.Kc, p.R);
@@ -1025,8 +1059,8 @@ int launch_dn_rows(const DnRowsParams& p, hipStream_t s) {
     hipLaunchKernelGGL(dn_conv_tail_kernel, dim3(cdiv(p.C, 256)), dim3(256), 0, s, p);
     TRX_LAUNCHED();
   }
-  const dim3 sg(p.nv, p.hv / rb);
-  const size_t lds = (size_t)2 * p.R * sizeof(float);
+  const dim3 sg(p.nv, cdiv(p.hv, kScanRows));
+  const size_t lds = (size_t)cdiv(p.R, kScanTile) * kScanTile * sizeof(float2);
   if (p.hk == 128) hipLaunchKernelGGL(dn_scan_kernel<128>, sg, dim3(256), lds, s, p);
   else hipLaunchKernelGGL(dn_scan_kernel<64>, sg, dim3(256), lds, s, p);
   TRX_LAUNCHED();
