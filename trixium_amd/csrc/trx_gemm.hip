@@ -17,12 +17,10 @@
 
 #include "trx_internal.h"
 #include "trx_prefill.h"
+#include "trx_rows_dev.h"
 
 namespace trx {
 
-typedef int i32x2_t __attribute__((ext_vector_type(2)));
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x8_t __attribute__((ext_vector_type(8)));
 typedef int i32x12_t __attribute__((ext_vector_type(12)));
 typedef unsigned int u32x6_t __attribute__((ext_vector_type(6)));
 typedef float f32x32_t __attribute__((ext_vector_type(32)));
@@ -172,138 +170,12 @@ int launch_planes(const PlanesParams& p, hipStream_t s) {
 
 // Weights ---------------------------------------------------------------------------------------
 
-// Code byte -> its weights as fp4: a trit5 byte's five nibbles (digit 0 first), a 2-bit byte's four
-// nibbles (twice). E2M1: 0 is 0, 1 is 2, 2 is 4, the sign is bit 3. Every entry is stored once per
-// LDS bank, so the 64 lanes' random bytes never conflict (one copy: 3.3 times the cycles).
-constexpr int kLut = 256 * 32;
+// A group's scale, 0 for a row past the end.
 template <int KIND>
-__device__ __forceinline__ void fill_lut(uint32_t* lut) {
-  auto nib = [](int c) { return c == 0 ? 0xAu : c == 1 ? 0u : c == 2 ? 2u : 4u; };
-  const int b = threadIdx.x >> 1, half = threadIdx.x & 1;    // 512 threads
-  uint32_t v = 0;
-  if (KIND == TRX_KIND_TERNARY5) {
-    int r = b;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      v |= nib(r % 3) << (4 * k);
-      r /= 3;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v |= nib((b >> (2 * k)) & 3) << (4 * k);
-    v |= v << 16;
-  }
-  uint4* d = (uint4*)(lut + 32 * b + 16 * half);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d[i] = make_uint4(v, v, v, v);
+__device__ __forceinline__ float row_scale(const RowReader<KIND>& row, const Codes& r) {
+  const float v = (float)__builtin_bit_cast(_Float16, (uint16_t)r.sc);
+  return row.valid ? v * kScaleUp : 0.f;
 }
-
-// The codes of one row's half group: 16 bytes from a dword boundary, and the group's scale.
-struct Codes {
-  i32x4_t c;
-  uint32_t sc;
-};
-
-template <int KIND>
-struct RowReader {
-  __amdgpu_buffer_rsrc_t rw;
-  uint32_t rbase, code_off;
-  int h;
-  bool valid;
-  __device__ __forceinline__ void init(const GemmParams& p, int r, int half) {
-    valid = r < p.M;
-    rw = make_rsrc(p.W, p.w_bytes);
-    rbase = (uint32_t)(valid ? r : 0) * (uint32_t)p.row_bytes;
-    code_off = (uint32_t)p.code_off;
-    h = half;
-  }
-  __device__ __forceinline__ uint32_t offset(int g) const {
-    return code_off + (KIND == TRX_KIND_TERNARY5 ? 26u * (uint32_t)g + 13u * (uint32_t)h
-                                                 : 32u * (uint32_t)g + 16u * (uint32_t)h);
-  }
-  __device__ __forceinline__ void load(Codes& r, int g) const {
-    r.c = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + (offset(g) & ~3u), 0, 0));
-    r.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
-  }
-  __device__ __forceinline__ float scale(const Codes& r) const {
-    const float v = (float)__builtin_bit_cast(_Float16, (uint16_t)r.sc);
-    return valid ? v * kScaleUp : 0.f;
-  }
-  // The 64 weights of the half group as fp4 in the planes' column order, in parts that a caller can
-  // spread over its other work: begin, look<0 .. 5> (the table reads of byte runs); low() and
-  // high() give the first and the second 32.
-  struct Half {
-    uint32_t d[4], p[KIND == TRX_KIND_TERNARY5 ? 13 : 16];
-  };
-  __device__ __forceinline__ void begin(const Codes& r, int g, Half& v) const {
-    if (KIND == TRX_KIND_TERNARY5) {
-      const uint32_t sh = offset(g) & 3u;
-      v.d[0] = __builtin_amdgcn_alignbyte(r.c[1], r.c[0], sh);
-      v.d[1] = __builtin_amdgcn_alignbyte(r.c[2], r.c[1], sh);
-      v.d[2] = __builtin_amdgcn_alignbyte(r.c[3], r.c[2], sh);
-      v.d[3] = __builtin_amdgcn_alignbyte(0, r.c[3], sh);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v.d[i] = (uint32_t)r.c[i];
-    }
-  }
-  template <int PART>
-  __device__ __forceinline__ void look(Half& v, const uint32_t* t) const {
-    constexpr int lo5[7] = {0, 2, 4, 6, 7, 10, 13}, lo2[7] = {0, 2, 4, 6, 8, 12, 16};
-    constexpr int a = KIND == TRX_KIND_TERNARY5 ? lo5[PART] : lo2[PART];
-    constexpr int b = KIND == TRX_KIND_TERNARY5 ? lo5[PART + 1] : lo2[PART + 1];
-#pragma unroll
-    for (int i = a; i < b; ++i) v.p[i] = t[((v.d[i >> 2] >> (8 * (i & 3))) & 0xFFu) * 32u];
-  }
-  // Holds the uses of the first (second) half's table values behind this point.
-  template <int HALF>
-  __device__ __forceinline__ void ready(Half& v) const {
-    uint32_t* p = v.p;
-    if constexpr (HALF == 0) {
-      asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7]));
-    } else {
-      asm volatile("" : "+v"(p[8]), "+v"(p[9]), "+v"(p[10]), "+v"(p[11]), "+v"(p[12]));
-      if constexpr (KIND == TRX_KIND_TERNARY) asm volatile("" : "+v"(p[13]), "+v"(p[14]), "+v"(p[15]));
-    }
-  }
-  __device__ __forceinline__ i32x4_t low(const Half& v) const {
-    const uint32_t* p = v.p;
-    if (KIND == TRX_KIND_TERNARY5)
-      return i32x4_t{(int)(p[0] | p[1] << 20), (int)(p[1] >> 12 | p[2] << 8 | p[3] << 28), (int)(p[3] >> 4 | p[4] << 16),
-                     (int)(p[4] >> 16 | p[5] << 4 | p[6] << 24)};
-    return i32x4_t{(int)two(p[0], p[1]), (int)two(p[2], p[3]), (int)two(p[4], p[5]), (int)two(p[6], p[7])};
-  }
-  __device__ __forceinline__ i32x4_t high(const Half& v) const {
-    const uint32_t* p = v.p;
-    if (KIND == TRX_KIND_TERNARY5) {
-      // Half 0's last byte ends with column 64, which half 1 takes after its own 63.
-      const auto sw = __builtin_amdgcn_permlane32_swap(p[12], p[12], false, false);
-      const uint32_t end = p[11] >> 4 | p[12] << 16;
-      return i32x4_t{(int)(p[6] >> 8 | p[7] << 12), (int)(p[8] | p[9] << 20), (int)(p[9] >> 12 | p[10] << 8 | p[11] << 28),
-                     (int)(h ? (end & 0x0FFFFFFFu) | (sw[0] >> 16) << 28 : end)};
-    }
-    return i32x4_t{(int)two(p[8], p[9]), (int)two(p[10], p[11]), (int)two(p[12], p[13]), (int)two(p[14], p[15])};
-  }
-  // Two 2-bit bytes' nibbles in one dword (a table entry holds its four nibbles twice).
-  __device__ __forceinline__ static uint32_t two(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
-  __device__ __forceinline__ void decode(const Codes& r, int g, const uint32_t* lut, uint32_t (&D)[8]) const {
-    const uint32_t* t = lut + (threadIdx.x & 31);
-    Half v;
-    begin(r, g, v);
-    look<0>(v, t);
-    look<1>(v, t);
-    look<2>(v, t);
-    look<3>(v, t);
-    look<4>(v, t);
-    look<5>(v, t);
-    const i32x4_t a = low(v), b = high(v);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      D[i] = (uint32_t)a[i];
-      D[4 + i] = (uint32_t)b[i];
-    }
-  }
-};
 
 // A step's digit planes of one position tile in registers: planes 0 and 1, 2 and 3, and 4 with the
 // block scales (dword 6) and the sum of squares (dword 7).
@@ -443,7 +315,7 @@ __device__ __forceinline__ void add_lone(const GemmParams& p, const PlaneReader&
     f32x16_t t = {};
     mx_lone_step(pl.load(2 * g), i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]}, t);
     mx_lone_step(pl.load(2 * g + 1), i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]}, t);
-    const float sc = row.scale(codes);
+    const float sc = row_scale<KIND>(row, codes);
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = fmaf(t[e], sc, acc[e]);
   }
@@ -498,14 +370,14 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
   Codes codes, next;                                  // the next group's, and the one after
   row.load(codes, 0);
   Planes q0 = pl.load(0), q1 = pl.load(1);
-  fill_lut<KIND>(lut);
+  fill_lut<KIND, true, kGmThreads>(lut);
   __syncthreads();
   {
     uint32_t D[8];
     row.decode(codes, 0, lut, D);
     bs[0][w][0][lane] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
     bs[0][w][1][lane] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
-    wsc[0][32 * w + j] = row.scale(codes);
+    wsc[0][32 * w + j] = row_scale<KIND>(row, codes);
     row.load(codes, min(1, G - 1));
     row.load(next, min(2, G - 1));
   }
@@ -578,7 +450,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
     TRX_SLOT(2, q1, t0, t1, x0, x1, t0, t1);
     s2 = wsc[buf][32 * (4 * ww + 2) + j];
     s3 = wsc[buf][32 * (4 * ww + 3) + j];
-    wsc[buf ^ 1][32 * w + j] = row.scale(codes);
+    wsc[buf ^ 1][32 * w + j] = row_scale<KIND>(row, codes);
     TRX_SLOT(3, q1, t0, t1, x0, x1, t0, t1);
     i32x4_t D1 = row.high(hv);
     TRX_PIN1(D1);
@@ -678,7 +550,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
 #pragma unroll
   for (int b = 0; b < NB; ++b) row[b].load(codes[b], gf);
   Planes q0 = pl.load(2 * gf), q1 = pl.load(2 * gf + 1);
-  fill_lut<KIND>(sm);
+  fill_lut<KIND, true, kGmThreads>(sm);
   __syncthreads();
   f32x16_t acc[NB] = {};
   float ss = 0.f;
@@ -693,7 +565,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
       row[b].decode(codes[b], g, sm, D);
       b0[b] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
       b1[b] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
-      sc[b] = row[b].scale(codes[b]);
+      sc[b] = row_scale<KIND>(row[b], codes[b]);
       row[b].load(codes[b], gn);
     }
     lone |= q0.scales() | q1.scales();

@@ -148,11 +148,19 @@ int gemv_f32(const uint8_t* rows, int kind, int M, int K, const float* x, const 
   return launch<TRX_KIND_TERNARY, MODE_F32>(p, s);
 }
 
+int gemv_exact_any(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int n, int B, int R, int32_t* y,
+                   int32_t* status, hipStream_t s);
+
 int gemv_exact(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int B, int R,
                int32_t* y, int32_t* status, hipStream_t s) {
   int rc = gemv_check(kind, M, K);
   if (rc) return rc;
   TRX_CHECK(x8 && y && status, TRX_E_INVALID, "gemv_exact: null argument");
+  // The matrix-core kernel (trx_gemv_rows.hip) below 2^25 weights, where its split of K over the waves and
+  // its small blocks win (6144 x 2048 7.3 -> 5.1 us, 2048 x 6144 2-bit 9.1 -> 6.0, 4096 x 4096 7.3 ->
+  // 5.8); above, this file's resident blocks (4096 x 12288 2-bit 9.95 against 10.5, 24576 x 4096 12.9
+  // against 13.9, 151936 x 4096 47.6 against 74.6).
+  if ((long long)M * K < (1ll << 25)) return gemv_exact_any(rows, kind, M, K, x8, 1, B, R, y, status, s);
   TRX_CHECK(B >= -48 && B <= 48 && R >= 0 && R < 63, TRX_E_INVALID, "gemv_exact: B=%d R=%d out of range", B, R);
   GemvParams p = {};
   fill_geom(p, rows, kind, M, K);

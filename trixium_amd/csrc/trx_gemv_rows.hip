@@ -1,230 +1,154 @@
-// Multi-row exact ternary GEMV: one pass over a tensor's row packets against up to kRowsMax
-// int8 activation vectors (model/bitexact.py:121-125 matvec_ternary_rows, the engine's
-// multi-row mode). Every output row is the single-row engine matvec of its x (per-group exact
-// sums, fp16 scale split, shift by e16 + B, int48 accumulate, >> R), bit for bit.
+// Exact engine matvec of one to eight int8 activation vectors (model/bitexact.py:101-125 matvec_ternary
+// and matvec_ternary_rows, the engine's op 0 and its multi-row mode) on the matrix cores: one pass
+// over a tensor's row packets. Every output is, bit for bit, per-group exact sums, the fp16 scale
+// split, the shift by e16 + B, the int48 accumulator and >> R.
 //
-// Layout of the work: a block (16 waves) stages all n x rows in LDS (n * K bytes); a wave owns a
-// weight row at a time. Its 64 lanes take 16 groups per pass, 4 lanes per 128-column group, lane
-// q holding columns 32q .. 32q+31 as eight dwords of int8 weights in {-1, 0, 1}:
-//   2-bit:  decoded from one 8-byte load;
-//   trit5:  lane q decodes code bytes 7q .. 7q+6 (columns 35q .. 35q+34, clipped to the group's
-//           26 bytes and 128 columns) into a per-wave LDS tile and reads its 32 columns back.
-// Each x row costs two 16-byte LDS reads and eight v_dot4_i32_i8 per lane; a quad shuffle gives
-// each group's exact sum, lane q = 0 shifts it into that row's int64 accumulator, and a wave
-// reduction ends the weight row.
+// A block takes 32 weight rows at a time and its waves split K. Per 128-column group and 32 rows a wave decodes the codes to int8 (a table read per code byte, a byte permute per four weights),
+// multiplies them by the x vectors with four v_mfma_i32_32x32x32_i8, multiplies the sums by the
+// scales' mantissas and adds them, shifted, to int64 accumulators; the waves' accumulators are added
+// through LDS (exact in any order). The x vectors take the first eight of the instruction's 32 rows
+// (vector r its row (r / 2) + 4 (r % 2), so that a lane holds every second vector's sum); the idle
+// rows cost nothing that bounds it, which is the weights' decode and, for small matrices, latency.
+// Measured against one v_dot4 pass per vector (up to four) or a v_dot4 pass over LDS-staged vectors:
+// eight vectors of a 6144 x 2048 trit5 matrix 18.3 -> 5.2 us, two of it 14.1 -> 5.3, one 7.3 -> 5.1.
 
 #include "trx_internal.h"
+#include "trx_rows_dev.h"
 
 namespace trx {
 
 int gemv_check(int kind, int M, int K);
 
-constexpr int kRowsThreads = 1024;
-constexpr int kRowsWaves = kRowsThreads / 64;
+typedef int i32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kRowsWaves = 8;
 constexpr int kRowsMax = 8;
-constexpr int kRowsTile = kRowsWaves * 16 * kGroup;   // decoded trit5 weights, 2 KiB per wave
-constexpr int kRowsLds = 144 * 1024 - kRowsTile;     // staged x rows: n * K bytes
+constexpr int kRowsStaged = 114688;    // n * K of a multi-row call
 
 struct RowsParams {
   const uint8_t* W;
-  const int8_t* x8;     // n rows of K int8, 16-byte aligned
+  uint32_t w_bytes;
+  const int8_t* x8;     // n rows of K int8
   int32_t* y;           // n rows of M int32
   int32_t* status;
-  int M, K, G, row_bytes, code_off, B, R;
+  int n, M, K, G, row_bytes, code_off, B, R;
 };
 
-template <int FMT, int NR>
-__global__ __launch_bounds__(kRowsThreads) void gemv_rows_kernel(RowsParams p) {
-  extern __shared__ __align__(16) int8_t xs[];
-  constexpr bool T5 = (FMT == TRX_KIND_TERNARY5);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j = lane >> 2, q = lane & 3;
-  // Per wave: 16 groups of decoded trit5 weights (int8 in {-1, 0, 1}), after the staged x rows.
-  int8_t* wd = xs + NR * p.K + wave * 16 * kGroup;
+// Eight codes (nibbles) as int8 weights: the even ones, the odd ones.
+__device__ __forceinline__ void weights8(uint32_t d, int& even, int& odd) {
+  constexpr uint32_t kW = 0x020100FFu;                // codes 0 .. 3: -1, 0, 1, 2
+  even = (int)__builtin_amdgcn_perm(kW, kW, d & 0x0F0F0F0Fu);
+  odd = (int)__builtin_amdgcn_perm(kW, kW, (d >> 4) & 0x0F0F0F0Fu);
+}
 
-  const int n16 = NR * p.K / 16;
-  for (int i = tid; i < n16; i += kRowsThreads) ((int4*)xs)[i] = ((const int4*)p.x8)[i];
+// E: sums per lane, half the vectors (rounded up). Few registers on purpose (up to eight waves a SIMD):
+// loads four groups ahead, tiles in turn over resident blocks, two tiles a wave and sixteen waves a
+// block all measured slower.
+template <int KIND, int E>
+__global__ __launch_bounds__(64 * kRowsWaves) void gemv_rows_kernel(RowsParams p) {
+  constexpr int W = kRowsWaves, kRed = W * 64 * E * 2;                // dwords of the waves' accumulators
+  __shared__ __align__(16) uint32_t sm[kRed > kLut ? kRed : kLut];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, j = lane & 31;
+  const int g0 = p.G * w / W, g1 = p.G * (w + 1) / W;
+  RowReader<KIND> row;
+  row.init(p, min(32 * (int)blockIdx.x + j, p.M), h);
+  // The vector of the instruction's row j; rows past the last vector repeat it (unread sums).
+  const int v = j < 8 ? 2 * (j & 3) + (j >> 2) : 0;
+  const int8_t* xr = p.x8 + (size_t)min(v, p.n - 1) * p.K + 64 * h;
+  Codes codes;
+  i32x4_t x[4];
+  auto load = [&](int g) {
+    row.load(codes, g);
+    // Any alignment: a single vector may start anywhere.
+#pragma unroll
+    for (int i = 0; i < 4; ++i) __builtin_memcpy(&x[i], xr + (size_t)kGroup * g + 16 * i, 16);
+  };
+  load(min(g0, p.G - 1));
+  fill_lut<KIND, false, 64 * W>(sm);
   __syncthreads();
-
-  for (int m = blockIdx.x * kRowsWaves + wave; m < p.M; m += gridDim.x * kRowsWaves) {
-    const uint8_t* row = p.W + (size_t)m * p.row_bytes;
-    const uint16_t* sc = (const uint16_t*)row;
-    long long acc[NR];
+  long long acc[E] = {};
+  for (int g = g0; g < g1; ++g) {
+    // x in the order of the decoded weights: from 65 on in half 1 of a trit5 group (64 last), the even
+    // columns of each eight, then the odd ones.
+    uint32_t d[16];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) acc[r] = 0;
-
-    for (int g0 = 0; g0 < p.G; g0 += 16) {
-      const int g = g0 + j;
-      const bool active = g < p.G;
-      // w[k]: this lane's columns 32q + 4k .. 32q + 4k + 3 as packed int8.
-      int w[8];
-      if (T5) {
-        // Lane q decodes code bytes 7q .. 7q+6 (columns 35q + 5i + d) into the wave's tile,
-        // then reads back its 32 aligned columns. The fence and wave barrier order the tile's
-        // writes before the reads of other lanes, and the previous pass's reads before them.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (active) {
-          const uint8_t* cb = row + p.code_off + (size_t)g * kTrit5GroupBytes;
-          int8_t* wg = wd + j * kGroup;
-#pragma unroll
-          for (int i = 0; i < 7; ++i) {
-            const int bi = 7 * q + i;
-            if (bi < kTrit5GroupBytes) {
-              unsigned t = cb[bi];
-#pragma unroll
-              for (int d = 0; d < 5; ++d) {
-                const int col = 5 * bi + d;
-                if (col < kGroup) wg[col] = (int8_t)((int)(t % 3u) - 1);
-                t /= 3u;
-              }
-            }
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (active) {
-          const int4* src = (const int4*)(wd + j * kGroup + 32 * q);
-          const int4 lo = src[0], hi = src[1];
-          w[0] = lo.x; w[1] = lo.y; w[2] = lo.z; w[3] = lo.w;
-          w[4] = hi.x; w[5] = hi.y; w[6] = hi.z; w[7] = hi.w;
-        }
-      } else if (active) {
-        const uint64_t v = *(const uint64_t*)(row + p.code_off + (size_t)g * kBeat + 8 * q);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          uint32_t d = 0;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            d |= (uint32_t)(uint8_t)(int8_t)((int)((v >> (8 * k + 2 * e)) & 3u) - 1) << (8 * e);
-          w[k] = (int)d;
-        }
-      }
-      int part[NR];
-#pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        int s = 0;
-        if (active) {
-          const int4* xr = (const int4*)(xs + r * p.K + g * kGroup + 32 * q);
-          const int4 lo = xr[0], hi = xr[1];
-          s = __builtin_amdgcn_sdot4(w[0], lo.x, s, false);
-          s = __builtin_amdgcn_sdot4(w[1], lo.y, s, false);
-          s = __builtin_amdgcn_sdot4(w[2], lo.z, s, false);
-          s = __builtin_amdgcn_sdot4(w[3], lo.w, s, false);
-          s = __builtin_amdgcn_sdot4(w[4], hi.x, s, false);
-          s = __builtin_amdgcn_sdot4(w[5], hi.y, s, false);
-          s = __builtin_amdgcn_sdot4(w[6], hi.z, s, false);
-          s = __builtin_amdgcn_sdot4(w[7], hi.w, s, false);
-        }
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        part[r] = s;
-      }
-      if (active && q == 0) {
-        int m11, e16;
-        fp16_split(sc[g], m11, e16);
-        const int sh = e16 + p.B;
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-          const long long prod = (long long)part[r] * (long long)m11;
-          long long c;
-          if (sh >= 0) c = prod << sh;
-          else c = (-sh >= 63) ? (prod < 0 ? -1 : 0) : (prod >> (-sh));
-          acc[r] += c;
-        }
-      }
+    for (int i = 0; i < 16; ++i) {
+      const uint32_t lo = (uint32_t)x[i >> 2][i & 3], hi = (uint32_t)x[((i + 1) & 15) >> 2][(i + 1) & 3];
+      d[i] = KIND == TRX_KIND_TERNARY5 ? __builtin_amdgcn_alignbyte(hi, lo, (uint32_t)h) : lo;
     }
-
+    i32x4_t a[4];
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      long long v = acc[r];
-#pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-      acc[r] = v;
+    for (int i = 0; i < 8; ++i) {
+      a[i >> 1][2 * (i & 1)] = (int)__builtin_amdgcn_perm(d[2 * i + 1], d[2 * i], 0x06040200u);
+      a[i >> 1][2 * (i & 1) + 1] = (int)__builtin_amdgcn_perm(d[2 * i + 1], d[2 * i], 0x07050301u);
     }
-    if (lane == 0) {
-      int bad = 0;
+    const Codes now = codes;
+    load(min(g + 1, g1 - 1));
+    uint32_t D[8];
+    row.decode(now, g, sm, D);
+    i32x16_t t = {};
 #pragma unroll
-      for (int r = 0; r < NR; ++r) {
-        const long long v = acc[r];
-        const long long res = v >> p.R;
-        bad |= ((v >= (1LL << 47)) || (v <= -(1LL << 47))) ? 1 : 0;
-        bad |= (res >= (1LL << 31) || res <= -(1LL << 31)) ? 2 : 0;
-        p.y[(size_t)r * p.M + m] = (int32_t)res;
-      }
-      if (bad) atomicOr(p.status, bad);
+    for (int s = 0; s < 4; ++s) {
+      int e0, o0, e1, o1;
+      weights8(D[2 * s], e0, o0);
+      weights8(D[2 * s + 1], e1, o1);
+      t = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s], i32x4_t{e0, o0, e1, o1}, t, 0, 0, 0);
     }
+    int m11, e16;
+    fp16_split((uint16_t)now.sc, m11, e16);
+    const int sh = e16 + p.B, left = max(sh, 0), right = min(max(-sh, 0), 63);
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] += ((long long)__mul24(t[e], m11) << left) >> right;
   }
+  long long* red = (long long*)sm;                    // [wave][e][lane]
+  __syncthreads();                                    // the table's reads are done
+#pragma unroll
+  for (int e = 0; e < E; ++e) red[(w * E + e) * 64 + lane] = acc[e];
+  __syncthreads();
+  if (w >= E) return;
+  const int r = 2 * w + h, m = 32 * (int)blockIdx.x + j;
+  if (r >= p.n || m >= p.M) return;
+  long long s = 0;
+#pragma unroll
+  for (int k = 0; k < W; ++k) s += red[(k * E + w) * 64 + lane];
+  const long long res = s >> p.R;
+  const int bad = (((s >= (1LL << 47)) || (s <= -(1LL << 47))) ? 1 : 0) |
+                  ((res >= (1LL << 31) || res <= -(1LL << 31)) ? 2 : 0);
+  p.y[(size_t)r * p.M + m] = (int32_t)res;
+  if (bad) atomicOr(p.status, bad);
 }
 
-static int rows_cus() {
-  static int n = 0;
-  if (!n) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    n = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-            ? prop.multiProcessorCount : 256;
-  }
-  return n;
-}
-
-template <int FMT, int NR>
+template <int KIND, int E>
 static int launch_rows(const RowsParams& p, hipStream_t s) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    TRX_HIP(hipFuncSetAttribute((const void*)gemv_rows_kernel<FMT, NR>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds + kRowsTile));
-    attr_set = true;
-  }
-  const int need = cdiv(p.M, kRowsWaves);
-  const int nb = need < rows_cus() ? need : rows_cus();
-  hipLaunchKernelGGL((gemv_rows_kernel<FMT, NR>), dim3(nb), dim3(kRowsThreads), NR * p.K + kRowsTile, s, p);
+  hipLaunchKernelGGL((gemv_rows_kernel<KIND, E>), dim3(cdiv(p.M, 32)), dim3(64 * kRowsWaves), 0, s, p);
   TRX_LAUNCHED();
   return TRX_OK;
 }
 
-template <int FMT>
-static int dispatch_rows(const RowsParams& p, int n, hipStream_t s) {
-  switch (n) {
-    case 1: return launch_rows<FMT, 1>(p, s);
-    case 2: return launch_rows<FMT, 2>(p, s);
-    case 3: return launch_rows<FMT, 3>(p, s);
-    case 4: return launch_rows<FMT, 4>(p, s);
-    case 5: return launch_rows<FMT, 5>(p, s);
-    case 6: return launch_rows<FMT, 6>(p, s);
-    case 7: return launch_rows<FMT, 7>(p, s);
-    default: return launch_rows<FMT, 8>(p, s);
+template <int KIND>
+static int dispatch_rows(const RowsParams& p, hipStream_t s) {
+  switch ((p.n + 1) / 2) {
+    case 1: return launch_rows<KIND, 1>(p, s);
+    case 2: return launch_rows<KIND, 2>(p, s);
+    case 3: return launch_rows<KIND, 3>(p, s);
+    default: return launch_rows<KIND, 4>(p, s);
   }
 }
 
-int gemv_exact(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int B, int R,
-               int32_t* y, int32_t* status, hipStream_t s);
-constexpr int kRowsSingleMax = 4;
-
-int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int n, int B,
-                    int R, int32_t* y, int32_t* status, hipStream_t s) {
-  TRX_CHECK(rows && x8 && y && status, TRX_E_INVALID, "gemv_exact_rows: null argument");
-  int rc = gemv_check(kind, M, K);
-  if (rc) return rc;
-  TRX_CHECK(n >= 1 && n <= kRowsMax, TRX_E_INVALID, "gemv_exact_rows: %d x rows (1..%d)", n, kRowsMax);
-  TRX_CHECK((long long)n * K <= kRowsLds, TRX_E_INVALID,
-            "gemv_exact_rows: %d x rows of K=%d exceed %d staged bytes", n, K, kRowsLds);
-  TRX_CHECK(((uintptr_t)x8 & 15) == 0, TRX_E_INVALID, "gemv_exact_rows: x8 must be 16-byte aligned");
-  TRX_CHECK(B >= -48 && B <= 48 && R >= 0 && R < 63, TRX_E_INVALID,
-            "gemv_exact_rows: B=%d R=%d out of range", B, R);
-  if (n <= kRowsSingleMax) {
-    // Few rows: the single-row kernel once per row is faster than one multi-row pass (measured at
-    // the 8B gate|up shape: 13.5 us a row against 34.5 us for a one-row pass, even at four rows).
-    for (int r = 0; r < n; ++r)
-      if ((rc = gemv_exact(rows, kind, M, K, x8 + (size_t)r * K, B, R, y + (size_t)r * M, status, s))) return rc;
-    return TRX_OK;
-  }
-  RowGeom rg = row_geom(kind, K);
+// n vectors (arguments checked by the callers).
+int gemv_exact_any(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int n, int B, int R, int32_t* y,
+                   int32_t* status, hipStream_t s) {
+  TRX_CHECK(B >= -48 && B <= 48 && R >= 0 && R < 63, TRX_E_INVALID, "gemv_exact: B=%d R=%d out of range", B, R);
+  const RowGeom rg = row_geom(kind, K);
   RowsParams p = {};
   p.W = rows;
+  // The last group of a row may be read up to 16 bytes past its end: the tensor is followed by a
+  // readable 32-byte tail.
+  p.w_bytes = (uint32_t)((unsigned long long)M * rg.row_bytes + 32);
   p.x8 = x8;
   p.y = y;
   p.status = status;
+  p.n = n;
   p.M = M;
   p.K = K;
   p.G = rg.G;
@@ -232,8 +156,19 @@ int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x
   p.code_off = rg.code_off;
   p.B = B;
   p.R = R;
-  if (kind == TRX_KIND_TERNARY5) return dispatch_rows<TRX_KIND_TERNARY5>(p, n, s);
-  return dispatch_rows<TRX_KIND_TERNARY>(p, n, s);
+  return kind == TRX_KIND_TERNARY5 ? dispatch_rows<TRX_KIND_TERNARY5>(p, s) : dispatch_rows<TRX_KIND_TERNARY>(p, s);
+}
+
+int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int n, int B,
+                    int R, int32_t* y, int32_t* status, hipStream_t s) {
+  TRX_CHECK(rows && x8 && y && status, TRX_E_INVALID, "gemv_exact_rows: null argument");
+  int rc = gemv_check(kind, M, K);
+  if (rc) return rc;
+  TRX_CHECK(n >= 1 && n <= kRowsMax, TRX_E_INVALID, "gemv_exact_rows: %d x rows (1..%d)", n, kRowsMax);
+  TRX_CHECK((long long)n * K <= kRowsStaged, TRX_E_INVALID,
+            "gemv_exact_rows: %d x rows of K=%d exceed %d bytes", n, K, kRowsStaged);
+  TRX_CHECK(((uintptr_t)x8 & 15) == 0, TRX_E_INVALID, "gemv_exact_rows: x8 must be 16-byte aligned");
+  return gemv_exact_any(rows, kind, M, K, x8, n, B, R, y, status, s);
 }
 
 }  // namespace trx
