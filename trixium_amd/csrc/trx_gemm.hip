@@ -241,6 +241,13 @@ __device__ __forceinline__ void mx_plane(const Planes& q, const i32x4_t (&w)[NB]
 #pragma unroll
   for (int b = 0; b < NB; ++b) t[b] = mx<C>(q, w[b], FIRST ? zero : t[b]);
 }
+// Keeps the products before it and the loads after it in place: the compiler otherwise moves every
+// load of a loop to its end, where its latency is waited out.
+template <int NB>
+__device__ __forceinline__ void pin(f32x16_t (&t)[NB]) {
+#pragma unroll
+  for (int i = 0; i < NB; ++i) asm volatile("" : "+v"(t[i]) : : "memory");
+}
 template <bool FIRST, int NB>
 __device__ __forceinline__ void mx_step(const Planes& q, const i32x4_t (&w)[NB], f32x16_t (&t)[NB]) {
   mx_plane<0, FIRST, NB>(q, w, t);
@@ -566,16 +573,20 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
       b0[b] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
       b1[b] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
       sc[b] = row_scale<KIND>(row[b], codes[b]);
+      asm volatile("" : "+v"(b0[b]), "+v"(b1[b]) : : "memory");
       row[b].load(codes[b], gn);
     }
     lone |= q0.scales() | q1.scales();
     f32x16_t t[NB];
-    mx_step<true, NB>(q0, b0, t);
     ss += q0.ss();
+    mx_step<true, NB>(q0, b0, t);
+    pin(t);
     q0 = pl.load(2 * gn);
-    mx_step<false, NB>(q1, b1, t);
     ss += q1.ss();
+    mx_step<false, NB>(q1, b1, t);
+    pin(t);
     q1 = pl.load(2 * gn + 1);
+    asm volatile("" : : : "memory");
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -646,9 +657,13 @@ static void gemm_ternary_kind(GemmParams& p, int nb, hipStream_t s) {
   p.nx = cdiv(tiles, nb);
   p.ny = cdiv(p.R, 32);
   const dim3 grid(p.nx * p.ny);
-  if (nb == 4) hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 4>), grid, dim3(kGmThreads), 0, s, p);
-  else if (nb == 2) hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 2>), grid, dim3(kGmThreads), 0, s, p);
-  else hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI == GM_SWIGLU ? GM_STORE : EPI, 1>), grid, dim3(kGmThreads), 0, s, p);
+  if (nb == 4) {
+    hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 4>), grid, dim3(kGmThreads), 0, s, p);
+  } else if (nb == 2) {
+    hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 2>), grid, dim3(kGmThreads), 0, s, p);
+  } else if constexpr (EPI != GM_SWIGLU) {             // SwiGLU takes a gate tile and its up tile
+    hipLaunchKernelGGL((gemm_split_kernel<KIND, EPI, 1>), grid, dim3(kGmThreads), 0, s, p);
+  }
 }
 
 template <int KIND>
@@ -671,13 +686,13 @@ int launch_gemm_ternary(const GemmParams& params, hipStream_t s) {
   TRX_HIP(hipGetDevice(&dev));
   TRX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   // The tile with the least estimated time: rounds of blocks over the CUs times a round's length, in
-  // us per 128 columns as measured at full rounds: 2.75 for the 128 x 256 tiles, 0.72, 0.46 and 0.36
-  // for the K-split tiles of 32 x 128, 64 and 32 (of 8, 4, 2 and 1 times the smallest's products per
+  // us per 128 columns as measured at one to twelve rounds: 2.75 for the 128 x 256 tiles, 0.65, 0.43 and
+  // 0.34 for the K-split tiles of 32 x 128, 64 and 32 (of 8, 4, 2 and 1 times the smallest's products per
   // wave's step: small tiles fill the chip on short prompts and narrow matrices only. 512 positions
-  // of a 2048 x 2048 matrix: 61 us in 32 large tiles, 25, 28 and 33 in 256, 512 and 1024 split ones;
-  // 2048 of a 24576 x 4096: 530 us against 1036).
+  // of a 2048 x 2048 matrix: 61 us in 32 large tiles, 23, 27 and 33 in 256, 512 and 1024 split ones;
+  // 2048 of a 24576 x 4096: 530 us against 930).
   const int tiles = p.epi == GM_SWIGLU ? 2 * cdiv(p.M / 2, 32) : cdiv(p.M, 32), npt = cdiv(p.R, 32);
-  const float len[4] = {2.75f, 0.72f, 0.46f, 0.36f};
+  const float len[4] = {2.75f, 0.65f, 0.43f, 0.34f};
   const int per[4] = {8, 4, 2, 1};
   int nb = 0;
   float best = 0.f;
