@@ -19,6 +19,8 @@
 #include "trx_prefill.h"
 #include "trx_rows_dev.h"
 
+#include <utility>
+
 namespace trx {
 
 typedef int i32x12_t __attribute__((ext_vector_type(12)));
@@ -351,190 +353,186 @@ __device__ __forceinline__ void tile_of_block(int b, int nx, int ny, int& x, int
 
 constexpr int kGmThreads = 512;
 
-// Large products: a block takes 128 positions x 256 weight rows. Wave w holds position tile w % 4
-// and weight tiles 4 (w / 4) .. + 3 (64 accumulator registers, 64 more for a group's sums); it loads
-// its positions' planes straight into registers (the operand order makes each load contiguous), most
-// of a group ahead of their use, and decodes one of the block's eight weight tiles per group into
-// LDS for all waves, two buffers, one barrier a group.
+// f with 0, 1, .. as compile-time constants.
+template <class F, int... I>
+__device__ __forceinline__ void in_turn(F f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>()), ...);
+}
+
+// Large products: a block takes 128 positions x 32 NT weight rows, four waves of one position tile
+// each, one wave a SIMD, so that a wave has 512 registers: NT accumulator tiles, the sums of two pairs
+// of tiles and two groups of its positions' planes, which it loads straight into registers a group
+// ahead of their use (the operand order makes each load contiguous). Each wave decodes NT / 4 of the block's
+// weight tiles per group into LDS for all, two buffers, one barrier a group.
 // A wave alone issues a vector operation every 6 cycles beside the matrix unit's 32-cycle products,
-// so all of a group's vector work (the last group's sums into the accumulators, the next group's
-// decode) is laid out between the products: 20 slots of two products and about ten operations.
-// 2048 positions of 24576 x 4096 with SwiGLU: 516 us (737 with fp16 planes), 2.7 us per group and
-// round against 1.7 for the products alone at the power-limited clock. The rest is every wave's own
-// copy of its planes (128 KB per group through the L1) and the table reads.
-template <int KIND, int EPI>
-__global__ __launch_bounds__(kGmThreads, 1) void gemm_kernel(GemmParams p) {
+// so all other work (the last pair's sums into the accumulators, the next group's decode, the loads)
+// is laid out between the products: slots of two products and about ten operations, ten a pair of tiles.
+// What vector operations touch (sums, accumulators) fills the 256 registers that they reach; planes and
+// weights lie in the others, which only products and loads reach.
+// Eight waves of four tiles each, at two waves a SIMD, read every plane twice as often and had no room for a
+// group ahead. 2048 positions, planes included: 24576 x 4096 with SwiGLU 503 us (520), 4096 x 12288 with the
+// residual 300 (333); 1024 of 34816 x 5120 491 (521). Per group and round 2.1 to 2.5 us, against 1.75 for the
+// products alone at the power-limited clock.
+template <int KIND, int EPI, int NT>
+__global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
+  constexpr int ND = NT / 4, NP = NT / 2;             // tiles a wave decodes, pairs
+  static_assert(NP % 2 == 0, "the pairs take turns with two sets of registers");
   __shared__ __align__(16) uint32_t lut[kLut];
-  __shared__ __align__(16) i32x4_t bs[2][8][2][64];
-  __shared__ float wsc[2][256];
+  __shared__ __align__(16) i32x4_t bs[2][NT][2][64];
+  __shared__ float wsc[2][32 * NT];
   __shared__ float rsx[128];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, j = lane & 31;
-  const int pw = w & 3, ww = w >> 2;
   int bx, by;
   tile_of_block(blockIdx.x, p.nx, p.ny, bx, by);
   const int G = p.K / kGroup, npt = (p.R + 31) / 32;
-  const int pt = min(4 * by + pw, npt - 1);           // a tile past the last repeats it, unstored
-  const bool live = 4 * by + pw < npt;
+  const int pt = min(4 * by + w, npt - 1);            // a tile past the last repeats it, unstored
+  const bool live = 4 * by + w < npt;
 
-  RowReader<KIND> row;
-  row.init(p, tile_row<EPI>(8 * bx + w, j, p.M), h);
+  RowReader<KIND> row[ND];
+  Codes codes[ND], next[ND];                          // the next group's, and the one after
   PlaneReader pl;
   pl.init(p, pt, lane);
-  Codes codes, next;                                  // the next group's, and the one after
-  row.load(codes, 0);
-  Planes q0 = pl.load(0), q1 = pl.load(1);
-  fill_lut<KIND, true, kGmThreads>(lut);
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    row[d].init(p, tile_row<EPI>(NT * bx + 4 * d + w, j, p.M), h);
+    row[d].load(codes[d], 0);
+  }
+  Planes qa0 = pl.load(0), qa1 = pl.load(1), qb0, qb1;
+  fill_lut<KIND, true, 256>(lut);
   __syncthreads();
-  {
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
     uint32_t D[8];
-    row.decode(codes, 0, lut, D);
-    bs[0][w][0][lane] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
-    bs[0][w][1][lane] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
-    wsc[0][32 * w + j] = row_scale<KIND>(row, codes);
-    row.load(codes, min(1, G - 1));
-    row.load(next, min(2, G - 1));
+    row[d].decode(codes[d], 0, lut, D);
+    bs[0][4 * d + w][0][lane] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
+    bs[0][4 * d + w][1][lane] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
+    wsc[0][32 * (4 * d + w) + j] = row_scale<KIND>(row[d], codes[d]);
+    row[d].load(codes[d], min(1, G - 1));
+    row[d].load(next[d], min(2, G - 1));
   }
   __syncthreads();
-  f32x16_t acc0 = {}, acc1 = {}, acc2 = {}, acc3 = {}, t0 = {}, t1 = {}, t2 = {}, t3 = {};
-  float ss = 0.f, s2 = 0.f, s3 = 0.f;
-  uint32_t lone = 0;
-  const i32x4_t (*fr)[2][64] = &bs[0][4 * ww];        // this wave's four tiles
-  i32x4_t x0 = fr[0][0][lane], x1 = fr[1][0][lane], y0, y1;
-  const f32x16_t zero = {};
-#define TRX_FMA(A, T, S, E0)                                                \
-  _Pragma("unroll") for (int e = E0; e < E0 + 8; ++e) A[e] = fmaf(T[e], S, A[e])
-#define TRX_SLOT(C, Q, TA, TB, XA, XB, CA, CB) \
-  TA = mx<C>(Q, XA, CA);                       \
-  TB = mx<C>(Q, XB, CB);                       \
-  asm volatile("" : "+v"(TA), "+v"(TB) : : "memory")
-#define TRX_PIN1(A) asm volatile("" : "+v"(A))
-  for (int g = 0; g < G; ++g) {
+  f32x16_t acc[NT] = {}, t[2][2] = {};
+  i32x4_t wt[2][2][2];                                // [pair's parity][step][tile]
+  float sc[2][2] = {}, ss = 0.f;
+  int lone = 0;
+  wt[0][0][0] = bs[0][0][0][lane];
+  wt[0][0][1] = bs[0][1][0][lane];
+  wt[0][1][0] = bs[0][0][1][lane];
+  wt[0][1][1] = bs[0][1][1][lane];
+  const uint32_t* lt = lut + (lane & 31);
+  typename RowReader<KIND>::Half hv;
+  // One slot: S of the group's 10 NP, the C-th of pair I, on planes q0, q1; the next group's go to n0, n1.
+  auto slot = [&](auto SC, int g, Planes& q0, Planes& q1, Planes& n0, Planes& n1) __attribute__((always_inline)) {
+    constexpr int S = decltype(SC)::value, I = S / 10, C = S % 10, ST = C / 5, T = I & 1, L = (I + NP - 1) % NP;
     const int buf = g & 1, gn = min(g + 1, G - 1);
-    const uint32_t n0 = pl.base(2 * gn), n1 = pl.base(2 * gn + 1);
-    const uint32_t* lt = lut + (lane & 31);
-    fr = &bs[buf][4 * ww];
-    lone |= q0.scales() | q1.scales();
-    // Step 0, tiles 0 and 1; the last group's tiles 2 and 3 into their accumulators.
-    y0 = fr[2][0][lane];
-    y1 = fr[3][0][lane];
-    ss += q0.ss();
-    ss += q1.ss();
-    TRX_SLOT(0, q0, t0, t1, x0, x1, zero, zero);
-    TRX_SLOT(1, q0, t0, t1, x0, x1, t0, t1);
-    TRX_FMA(acc2, t2, s2, 0);
-    TRX_PIN1(acc2);
-    TRX_SLOT(2, q0, t0, t1, x0, x1, t0, t1);
-    TRX_FMA(acc2, t2, s2, 8);
-    TRX_PIN1(acc2);
-    TRX_SLOT(3, q0, t0, t1, x0, x1, t0, t1);
-    TRX_FMA(acc3, t3, s3, 0);
-    TRX_PIN1(acc3);
-    TRX_SLOT(4, q0, t0, t1, x0, x1, t0, t1);
-    TRX_FMA(acc3, t3, s3, 8);
-    TRX_PIN1(acc3);
-    // Step 0, tiles 2 and 3; the planes' registers take the next group's; the codes' first half.
-    typename RowReader<KIND>::Half hv;
-    row.begin(codes, gn, hv);
-    x0 = fr[0][1][lane];
-    x1 = fr[1][1][lane];
-    TRX_SLOT(0, q0, t2, t3, y0, y1, zero, zero);
-    row.template look<0>(hv, lt);
-    TRX_SLOT(1, q0, t2, t3, y0, y1, t2, t3);
-    q0.c01 = pl.pair(n0, 0);
-    row.template look<1>(hv, lt);
-    TRX_SLOT(2, q0, t2, t3, y0, y1, t2, t3);
-    row.template look<2>(hv, lt);
-    TRX_SLOT(3, q0, t2, t3, y0, y1, t2, t3);
-    q0.c23 = pl.pair(n0, 3);
-    row.template look<3>(hv, lt);
-    TRX_SLOT(4, q0, t2, t3, y0, y1, t2, t3);
-    q0.c4 = pl.last(n0);
-    i32x4_t D0 = row.low(hv);
-    TRX_PIN1(D0);
-    // Step 1, tiles 0 and 1; the codes' second half.
-    y0 = fr[2][1][lane];
-    y1 = fr[3][1][lane];
-    TRX_SLOT(0, q1, t0, t1, x0, x1, t0, t1);
-    bs[buf ^ 1][w][0][lane] = D0;
-    row.template look<4>(hv, lt);
-    TRX_SLOT(1, q1, t0, t1, x0, x1, t0, t1);
-    row.template look<5>(hv, lt);
-    const float s0 = wsc[buf][32 * (4 * ww) + j], s1 = wsc[buf][32 * (4 * ww + 1) + j];
-    TRX_SLOT(2, q1, t0, t1, x0, x1, t0, t1);
-    s2 = wsc[buf][32 * (4 * ww + 2) + j];
-    s3 = wsc[buf][32 * (4 * ww + 3) + j];
-    wsc[buf ^ 1][32 * w + j] = row_scale<KIND>(row, codes);
-    TRX_SLOT(3, q1, t0, t1, x0, x1, t0, t1);
-    i32x4_t D1 = row.high(hv);
-    TRX_PIN1(D1);
-    TRX_SLOT(4, q1, t0, t1, x0, x1, t0, t1);
-    bs[buf ^ 1][w][1][lane] = D1;
-    codes = next;
-    row.load(next, min(g + 3, G - 1));
-    // Step 1, tiles 2 and 3; after the barrier the next group's first weights.
-    TRX_SLOT(0, q1, t2, t3, y0, y1, t2, t3);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    fr = &bs[buf ^ 1][4 * ww];
-    x0 = fr[0][0][lane];
-    x1 = fr[1][0][lane];
-    TRX_SLOT(1, q1, t2, t3, y0, y1, t2, t3);
-    q1.c01 = pl.pair(n1, 0);
-    TRX_FMA(acc0, t0, s0, 0);
-    TRX_PIN1(acc0);
-    TRX_SLOT(2, q1, t2, t3, y0, y1, t2, t3);
-    TRX_FMA(acc0, t0, s0, 8);
-    TRX_PIN1(acc0);
-    TRX_SLOT(3, q1, t2, t3, y0, y1, t2, t3);
-    q1.c23 = pl.pair(n1, 3);
-    TRX_FMA(acc1, t1, s1, 0);
-    TRX_PIN1(acc1);
-    TRX_SLOT(4, q1, t2, t3, y0, y1, t2, t3);
-    q1.c4 = pl.last(n1);
-    TRX_FMA(acc1, t1, s1, 8);
-    TRX_PIN1(acc1);
+    const f32x16_t zero = {};
+    Planes& q = ST ? q1 : q0;
+    if constexpr (I == 0 && C % 5 == 0) asm volatile("" : "+a"(q.c01));
+    if constexpr (I == 0 && C % 5 == 2) asm volatile("" : "+a"(q.c23));
+    if constexpr (I == 0 && C % 5 == 4) asm volatile("" : "+a"(q.c4));
+    t[T][0] = mx<C % 5>(q, wt[T][ST][0], C ? t[T][0] : zero);
+    t[T][1] = mx<C % 5>(q, wt[T][ST][1], C ? t[T][1] : zero);
+    asm volatile("" : "+v"(t[T][0]), "+v"(t[T][1]) : : "memory");
+    if constexpr (S == 4 || S == 9) {
+      lone |= __any((int)q.scales() < 0);
+      ss += q.ss();
+      asm volatile("" : "+a"(ss));
+    }
+    // The last pair's sums, four a slot.
+    if constexpr (C >= 1 && C <= 8) {
+      constexpr int k = (C - 1) / 4, e0 = 4 * ((C - 1) % 4);
+#pragma unroll
+      for (int e = e0; e < e0 + 4; ++e) acc[2 * L + k][e] = fmaf(t[T ^ 1][k][e], sc[T ^ 1][k], acc[2 * L + k][e]);
+      asm volatile("" : "+v"(acc[2 * L + k]));
+    }
+    // The next group's planes, in six parts, a step's scales first.
+    if constexpr (S % 3 == 0 && S < 18) {
+      constexpr int k = S / 3;
+      Planes& n = k < 3 ? n0 : n1;
+      const uint32_t b = pl.base(2 * gn + k / 3);
+      if constexpr (k % 3 == 0) n.c4 = pl.last(b);
+      else if constexpr (k % 3 == 1) n.c01 = pl.pair(b, 0);
+      else n.c23 = pl.pair(b, 3);
+    }
+    // The next pair's weights: the next group's for the last pair, behind the barrier.
+    if constexpr (I == NP - 1) {
+      if constexpr (C == 4) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if constexpr (C == 4 || C == 6) {
+        wt[T ^ 1][(C - 4) / 2][0] = bs[buf ^ 1][0][(C - 4) / 2][lane];
+        wt[T ^ 1][(C - 4) / 2][1] = bs[buf ^ 1][1][(C - 4) / 2][lane];
+      }
+    } else if constexpr (C == 2 || C == 4) {
+      wt[T ^ 1][(C - 2) / 2][0] = bs[buf][2 * I + 2][(C - 2) / 2][lane];
+      wt[T ^ 1][(C - 2) / 2][1] = bs[buf][2 * I + 3][(C - 2) / 2][lane];
+    }
+    if constexpr (C == 3) {
+      sc[T][0] = wsc[buf][32 * (2 * I) + j];
+      sc[T][1] = wsc[buf][32 * (2 * I + 1) + j];
+    }
+    // The next group's decode: a tile over two pairs.
+    constexpr int d = I / 2, o = S % 20;
+    if constexpr (o == 0) row[d].begin(codes[d], gn, hv);
+    if constexpr (o <= 3) row[d].template look<o <= 3 ? o : 0>(hv, lt);
+    if constexpr (o == 6) bs[buf ^ 1][4 * d + w][0][lane] = row[d].low(hv);
+    if constexpr (o == 7 || o == 8) row[d].template look<o == 7 ? 4 : 5>(hv, lt);
+    if constexpr (o == 9) wsc[buf ^ 1][32 * (4 * d + w) + j] = row_scale<KIND>(row[d], codes[d]);
+    if constexpr (o == 12) {
+      bs[buf ^ 1][4 * d + w][1][lane] = row[d].high(hv);
+      codes[d] = next[d];
+      asm volatile("" : "+a"(row[d].rbase), "+a"(row[d].h));          // or its sums with the offsets spill
+      row[d].load_uniform(next[d], min(g + 3, G - 1));
+    }
+  };
+  auto group = [&](int g, Planes& q0, Planes& q1, Planes& n0, Planes& n1) __attribute__((always_inline)) {
+    in_turn([&](auto S) __attribute__((always_inline)) { slot(S, g, q0, q1, n0, n1); },
+            std::make_integer_sequence<int, 10 * NP>());
+  };
+  for (int g = 0; g < G; g += 2) {
+    group(g, qa0, qa1, qb0, qb1);
+    if (g + 1 == G) break;
+    group(g + 1, qb0, qb1, qa0, qa1);
   }
-  TRX_FMA(acc2, t2, s2, 0);
-  TRX_FMA(acc2, t2, s2, 8);
-  TRX_FMA(acc3, t3, s3, 0);
-  TRX_FMA(acc3, t3, s3, 8);
-  if (__any((int)lone < 0)) {
-    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww, lut, 0, G, acc0);
-    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 1, lut, 0, G, acc1);
-    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 2, lut, 0, G, acc2);
-    add_lone<KIND, EPI>(p, pl, 8 * bx + 4 * ww + 3, lut, 0, G, acc3);
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[NT - 2 + k][e] = fmaf(t[1][k][e], sc[1][k], acc[NT - 2 + k][e]);
+  if (lone) {
+#pragma unroll
+    for (int b = 0; b < NT; ++b) add_lone<KIND, EPI>(p, pl, NT * bx + b, lut, 0, G, acc[b]);
   }
-#undef TRX_FMA
-#undef TRX_SLOT
-#undef TRX_PIN1
 
   // Accumulator e of lane l holds position i = 8 (e / 4) + 4 (l / 32) + e % 4, weight row l % 32.
-  if (ww == 0) {
-    ss += __shfl_xor(ss, 32, 64);
-    if (h == 0) rsx[32 * pw + j] = p.norm ? 1.0f / sqrtf(ss / (float)p.K + p.eps) : 1.f;
-  }
+  ss += __shfl_xor(ss, 32, 64);
+  if (h == 0) rsx[32 * w + j] = p.norm ? 1.0f / sqrtf(ss / (float)p.K + p.eps) : 1.f;
   __syncthreads();
   if (!live) return;
+  // Four positions' residuals are read before the first is used: one at a time each waits for memory
+  // (128 of them, 30 us a block).
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int i = 8 * (e >> 2) + 4 * h + (e & 3), r = 32 * pt + i;
-    if (r >= p.R) continue;
-    const float rs = rsx[32 * pw + i];
-    float* yr = p.y + (size_t)r * p.ldy;
-    const float v[4] = {acc0[e] * rs, acc1[e] * rs, acc2[e] * rs, acc3[e] * rs};
-    if (EPI == GM_SWIGLU) {
+  for (int e0 = 0; e0 < 16; e0 += 4) {
+    const int i0 = 2 * e0 + 4 * h, r0 = 32 * pt + i0;
+    float old[4][NT] = {};
+    if (EPI == GM_RESID) {
 #pragma unroll
-      for (int b = 0; b < 4; b += 2) {
-        const int f = 32 * ((8 * bx + 4 * ww + b) >> 1) + j;
-        if (f < p.M / 2) yr[f] = silu(v[b]) * v[b + 1];
-      }
-    } else {
+      for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int m = 32 * (8 * bx + 4 * ww + b) + j;
-        if (m < p.M) {
-          if (EPI == GM_RESID) yr[m] += v[b];
-          else yr[m] = v[b];
+        for (int b = 0; b < NT; ++b) {
+          const int m = 32 * (NT * bx + b) + j;
+          if (r0 + k < p.R && m < p.M) old[k][b] = p.y[(size_t)(r0 + k) * p.ldy + m];
         }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float rs = rsx[32 * w + i0 + k];
+      float* yr = p.y + (size_t)(r0 + k) * p.ldy;
+#pragma unroll
+      for (int b = 0; b < NT; b += EPI == GM_SWIGLU ? 2 : 1) {
+        const int m = EPI == GM_SWIGLU ? 32 * ((NT * bx + b) >> 1) + j : 32 * (NT * bx + b) + j;
+        if (r0 + k >= p.R || m >= (EPI == GM_SWIGLU ? p.M / 2 : p.M)) continue;
+        const float v = acc[b][e0 + k] * rs;
+        if constexpr (EPI == GM_SWIGLU) yr[m] = silu(v) * (acc[b + 1][e0 + k] * rs);
+        else if (EPI == GM_RESID) yr[m] = old[k][b] + v;
+        else yr[m] = v;
       }
     }
   }
@@ -659,7 +657,7 @@ static void gemm_ternary_kind(GemmParams& p, int nb, hipStream_t s) {
   if (nb == 0) {
     p.nx = cdiv(tiles, 8);
     p.ny = cdiv(p.R, 128);
-    hipLaunchKernelGGL((gemm_kernel<KIND, EPI>), dim3(p.nx * p.ny), dim3(kGmThreads), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<KIND, EPI, 8>), dim3(p.nx * p.ny), dim3(256), 0, s, p);
     return;
   }
   p.nx = cdiv(tiles, nb);
@@ -694,13 +692,13 @@ int launch_gemm_ternary(const GemmParams& params, hipStream_t s) {
   TRX_HIP(hipGetDevice(&dev));
   TRX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   // The tile with the least estimated time: rounds of blocks over the CUs times a round's length, in
-  // us per 128 columns as measured at one to twelve rounds: 2.75 for the 128 x 256 tiles, 0.65, 0.43 and
+  // us per 128 columns as measured at one to twelve rounds: 2.55 for the 128 x 256 tiles, 0.65, 0.43 and
   // 0.34 for the K-split tiles of 32 x 128, 64 and 32 (of 8, 4, 2 and 1 times the smallest's products per
   // wave's step: small tiles fill the chip on short prompts and narrow matrices only. 512 positions
   // of a 2048 x 2048 matrix: 61 us in 32 large tiles, 23, 27 and 33 in 256, 512 and 1024 split ones;
-  // 2048 of a 24576 x 4096: 530 us against 930).
+  // 2048 of a 24576 x 4096: 503 us against 930).
   const int tiles = p.epi == GM_SWIGLU ? 2 * cdiv(p.M / 2, 32) : cdiv(p.M, 32), npt = cdiv(p.R, 32);
-  const float len[4] = {2.75f, 0.65f, 0.43f, 0.34f};
+  const float len[4] = {2.55f, 0.65f, 0.43f, 0.34f};
   const int per[4] = {8, 4, 2, 1};
   int nb = 0;
   float best = 0.f;

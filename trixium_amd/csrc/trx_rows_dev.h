@@ -66,6 +66,14 @@ struct RowReader {
     r.c = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + (offset(g) & ~3u), 0, 0));
     r.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
   }
+  // load() of a group that is the same for the wave: its product stays scalar (as one multiply-add with
+  // the row's offset it keeps a 64-bit register pair).
+  __device__ __forceinline__ void load_uniform(Codes& r, int g) const {
+    uint32_t at = (KIND == TRX_KIND_TERNARY5 ? 26u : 32u) * (uint32_t)g;
+    asm("" : "+s"(at));
+    r.c = __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, rbase + ((offset(0) + at) & ~3u), 0, 0));
+    r.sc = __builtin_amdgcn_raw_buffer_load_b16(rw, rbase + 2u * (uint32_t)g, 0, 0);
+  }
   // The 64 weights of the half group as nibbles, in the columns' order (trit5: half 1 takes columns 65 ..
   // 127 and then 64, whose code shares a byte with half 0's), in parts that a caller can
   // spread over its other work: begin, look<0 .. 5> (the table reads of byte runs); low() and
