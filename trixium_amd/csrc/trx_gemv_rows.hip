@@ -166,7 +166,7 @@ int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x
   if (rc) return rc;
   TRX_CHECK(n >= 1 && n <= kRowsMax, TRX_E_INVALID, "gemv_exact_rows: %d x rows (1..%d)", n, kRowsMax);
   TRX_CHECK((long long)n * K <= kRowsStaged, TRX_E_INVALID,
-            "gemv_exact_rows: %d x rows of K=%d exceed %d bytes", n, K, kRowsStaged);
+            "gemv_exact_rows: %d x rows of K=%d exceed %d staged bytes", n, K, kRowsStaged);
   TRX_CHECK(((uintptr_t)x8 & 15) == 0, TRX_E_INVALID, "gemv_exact_rows: x8 must be 16-byte aligned");
   return gemv_exact_any(rows, kind, M, K, x8, n, B, R, y, status, s);
 }
