@@ -1,8 +1,8 @@
 """The ternary GEMM's digit planes and tile shapes on the GPU (trx_gemm.hip), against float64.
 
-The bound is derived: what the five digits leave of x is at most half an ulp of its 32-column block's
-largest value (2^-24 of it; 2^-105 where the block lies below 2^-80, the smallest exponent), a
-group's ten matrix instructions and the sums over the G groups round in float32 (2^-24 of the partial
+The bound is derived: what the five digits leave of x is at most 2^-23 of its own leading power or 2^-25
+of its 32-column block's, whichever is more (2^-106 where the block lies below 2^-80, the smallest
+exponent): 2^-24 of the largest value plus two of the sums' half units cover both. A group's ten matrix instructions and the sums over the G groups round in float32 (2^-24 of the partial
 sums each, which the sum of |w x| bounds), and the output adds a few roundings (the RMSNorm's scale,
 the residual). Up to three values 2^7 or more above the rest of their block do not count as its
 largest.
@@ -139,3 +139,51 @@ def test_lone_values_keep_the_rest(kind, M, n):
             x[r, col] = f * x[r, at[r]]
             rest[r, col] = abs(x[r, at[r]])          # they share a scale of their own
     _check(kind, M, K, n, _lib.EPI_STORE, False, x.astype(np.float32), rng, top=rest)
+
+
+def _fp16_pair(x):
+    """x as a float32 sum of two fp16 values of its row's scale (what the kernel's predecessor multiplied)."""
+    xs = 2.0 ** np.maximum(0, np.frexp(np.abs(x).max(axis=1, keepdims=True))[1] - 14)
+    y = (x / xs).astype(np.float32)
+    hi = y.astype(np.float16).astype(np.float32)
+    return ((hi + (y - hi).astype(np.float16).astype(np.float32)) * xs).astype(np.float64)
+
+
+# Inputs as projections meet them: a normed residual stream with and without larger channels, products of
+# two normals, SwiGLU activations.
+def _inputs(name, n, K, rng):
+    x = rng.standard_normal((n, K))
+    if name == "channels":
+        x[:, rng.permutation(K)[:K // 512]] *= 20
+    elif name == "product":
+        x *= rng.standard_normal((n, K))
+    elif name == "swiglu":
+        x *= (lambda g: g / (1 + np.exp(-g)))(3 * rng.standard_normal((n, K)))
+    elif name == "large":
+        x *= 100
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
+@pytest.mark.parametrize("name", ["normal", "channels", "product", "swiglu", "large"])
+@pytest.mark.parametrize("M,n", [(512, 200), (8192, 1100)])
+def test_operands(kind, name, M, n):
+    """Weights of one trit a row and scale 1 hand x back as the products see it. Every value is held to 2^-23 of
+    its own leading power or 2^-25 of its block's, whichever is more (half 1 of a trit5 group takes its columns one
+    later: the bound takes the 128-column group's), and the sum rounds to float32 (two half units); over all
+    values the error is no larger than that of a pair of fp16 values."""
+    rng = np.random.default_rng(M + n + len(name))
+    K = 512
+    codes = np.ones((M, K), np.uint8)
+    codes[np.arange(M), np.arange(M) % K] = 2
+    rows = encode_rows(kind, K, np.ones((M, K // 128), np.float16), codes)
+    x = _inputs(name, n, K, rng)
+    got = _run(rows, kind, M, K, x, None, _lib.EPI_STORE, None).reshape(n, M // K, K)
+    assert np.array_equal(got, np.broadcast_to(got[:, :1], got.shape))
+    v = x.astype(np.float64)
+    err, lead = np.abs(got[:, 0] - v), 2.0 ** (np.frexp(v)[1] - 1)
+    top = lead.reshape(n, K // 128, 128).max(axis=2).repeat(128, axis=1)
+    assert np.all(err <= np.maximum(2.0**-23 * lead, 2.0**-25 * top) + 2.0**-23 * lead)
+    rms = [float(np.sqrt(np.mean(e * e))) for e in (err, _fp16_pair(x) - v)]
+    print(f"{name} rms error {rms[0]:.2e}, of an fp16 pair {rms[1]:.2e}", flush=True)
+    assert rms[0] <= rms[1]

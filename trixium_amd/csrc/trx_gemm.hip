@@ -1,15 +1,17 @@
 // The ternary GEMM of several positions on the matrix cores: y[r] = W xhat_r.
 //
-// x enters as five planes of base-32 digits in fp6 (E2M3), W's trits as fp4 (E2M1), so that the
-// products run on v_mfma_scale_f32_32x32x64_f8f6f4 at its fp6/fp4 rate, four times fp16's:
-//   x = 2^u (d0 + d1/32 + d2/32^2 + d3/32^3 + d4/32^4), every digit a whole number in [-16, 16]
-// with one exponent u per position and 32 columns (the largest |x| in [8, 16) * 2^u, but see Lone). E2M3 holds
-// every whole number of eighths up to 16 exactly and E2M1 holds -1, 0, 1 (and 2, the 2-bit code
-// 3) exactly, the plane's power of two is the instruction's block scale, and its fp32 accumulation
-// of such products is exact while a sum fits 24 bits. What is left of x is at most 2^(u - 21): half
-// an ulp of the block's largest value. A group's sum is then multiplied by the group's fp16 scale
-// and added in fp32, so the result is nearer to the exact one than fp32 products added one by one
-// (against float64, K = 4096: 2e-7 of the result's norm; two fp16 planes gave 6e-7).
+// x enters as five planes of digits in fp6 (E2M3), W's trits as fp4 (E2M1), so that the products run on
+// v_mfma_scale_f32_32x32x64_f8f6f4 at its fp6/fp4 rate, four times fp16's:
+//   x = 2^u (d0 + d1/2^5 + d2/2^10 + d3/2^15 + d4/2^21), every digit a whole number of the format's eighths
+// with one exponent u per position and 32 columns (the largest |x| in [16, 32) * 2^u, but see Lone). E2M3 holds
+// whole eighths up to 2, every second one up to 4 and every fourth up to 7.5, and E2M1 holds -1, 0, 1 (and 2,
+// the 2-bit code 3); the plane's power of two is the instruction's block scale, and its fp32 accumulation of
+// such products is exact while a sum fits 24 bits. A value of the block's highest octave leaves up to four
+// units of the next digit, any other two. So the last digit, a bit further down, holds the others to 2^(u - 21)
+// (2^-25 of the block's leading power) and the highest octave's, whose last digit ends at 7.5 where 8 is due,
+// to 2^(u - 19) (2^-23 of its own). Over normed, SwiGLU and attention inputs that is a smaller error than a
+// pair of fp16 values has (root mean square 2.2e-8 against 4.5e-8 for normal x; the last digit at 2^20 and the
+// largest |x| in [8, 16) * 2^u: 6.6e-8). A group's sum is then multiplied by the group's fp16 scale and added in fp32.
 // Measured on all CUs (operands in registers, random data): 6.1 PFLOP/s for fp6 x fp4, 3.4 for
 // int8, 1.57 for fp16; with the planes that each needs for fp32-accurate x (5, 3, 2) that is 1.23,
 // 1.14 and 0.79 PFLOP/s, and the int8 planes' sums would need five vector operations per element
@@ -37,11 +39,13 @@ typedef float f32x32_t __attribute__((ext_vector_type(32)));
 // lowest digit's first), then the block's scales and the fp32 sum of the 32 columns' x^2. Four bytes a column in all, read by 16-byte loads only (per byte, the
 // vector cache is a quarter slower on 8- and 12-byte ones).
 constexpr int kPlanes = 5;
-constexpr int kUMin = -84;             // smallest u: below it values lose bits under 2^-109
+constexpr int kUMin = -85;             // smallest u: below it values lose bits under 2^-106
 constexpr int kApart = 7;
 // The block scales hold the planes 2^16 down and the weights' scales 2^16 up, so that no group's sum
 // of finite values overflows.
-constexpr int kScaleByte = 110 - 16;
+constexpr int kScaleByte = 109 - 16;
+// Plane c's power of two above plane 0's.
+constexpr uint32_t plane_up(int c) { return c ? 5 * c + 1 : 0; }
 constexpr float kScaleUp = 65536.f;
 
 // A lane packs one position's 32 columns with the hardware's fp6 conversions (digit by digit in floats it
@@ -103,7 +107,7 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
   }
   const bool finite = top < 0x7F800000u;
   // One to three values 2^kApart or more above the rest (see Lone values below): the block's exponent is
-  // the rest's, and they go in 2^-apart times. u from an exponent field E: E - 130.
+  // the rest's, and they go in 2^-apart times. u from an exponent field E: E - 131.
   const uint32_t high = top > ((uint32_t)kApart << 23) ? top - ((uint32_t)kApart << 23) : 0;
   uint32_t rest = 0;
   int count = 0;
@@ -113,10 +117,10 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
     count += (ma >= high) + (mb >= high);
     rest = max(rest, max(ma >= high ? 0u : ma, mb >= high ? 0u : mb));
   }
-  int u = max((int)(top >> 23) - 130, kUMin), apart = 0;
+  int u = max((int)(top >> 23) - 131, kUMin), apart = 0;
   uint32_t where = 0;
   if (finite && rest != 0 && count <= 3) {
-    const int un = max((int)(rest >> 23) - 130, kUMin);
+    const int un = max((int)(rest >> 23) - 131, kUMin);
     apart = u - un;
     u = un;
     auto lone = [&](float x, int e) {
@@ -136,7 +140,8 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
   uint32_t dw[32];
 #pragma unroll
   for (int d = 0; d < kPlanes; ++d) {
-    const float sc = __uint_as_float((uint32_t)(u + 3 - 5 * d + 127) << 23);
+    const int c = kPlanes - 1 - d;
+    const float sc = __uint_as_float((uint32_t)(u + 3 - 21 + (int)plane_up(c) + 127) << 23);
     const u32x6_t q = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, sc);
     // The sources stay live past the conversion: it reads them while it writes its result, and the
     // compiler may otherwise give both the same registers.
@@ -151,9 +156,9 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
       }
     }
 #pragma unroll
-    for (int i = 0; i < 6; ++i) dw[6 * (kPlanes - 1 - d) + i] = q[i];
+    for (int i = 0; i < 6; ++i) dw[6 * c + i] = q[i];
   }
-  // Byte 0: the block scale of the lowest plane (plane c's is 5 c above); 0xFF, the format's NaN, where a
+  // Byte 0: the block scale of the lowest plane (plane c's is plane_up(c) above); 0xFF, the format's NaN, where a
   // value is not finite. Byte 1: the lone values' shift; then their three places and bit 31.
   dw[30] = !finite ? 0xFFu
                    : (uint32_t)(u + kScaleByte) | (apart > 0 ? (uint32_t)apart << 8 | where << 16 | 0x80000000u : 0u);
@@ -235,7 +240,7 @@ struct PlaneReader {
 template <int C>
 __device__ __forceinline__ f32x16_t mx(const Planes& q, const i32x4_t& w, const f32x16_t& acc) {
   const i32x8_t B = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
-  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(q.get<C>(), B, acc, 2, 4, 0, (int)(q.scales() + 5u * C), 0,
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(q.get<C>(), B, acc, 2, 4, 0, (int)(q.scales() + plane_up(C)), 0,
                                                           0x7F7F7F7F);
 }
 
@@ -298,7 +303,7 @@ __device__ __forceinline__ f32x16_t mx_lone(const Planes& q, const i32x4_t& w, f
     N[i] = A[i] ^ (int)sign;
   }
   const i32x8_t B = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
-  const uint32_t s0 = (s & 0xFFu) + 5u * C;
+  const uint32_t s0 = (s & 0xFFu) + plane_up(C);
   acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(N, B, acc, 2, 4, 0, (int)s0, 0, 0x7F7F7F7F);
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, acc, 2, 4, 0, (int)(s0 + (on ? s >> 8 & 0xFFu : 0u)), 0,
                                                           0x7F7F7F7F);
