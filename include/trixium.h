@@ -111,11 +111,15 @@ int trx_gemv_ternary_f32(const uint8_t* rows, int kind, int M, int K, const floa
 /* Multi-position float projection, the batched prefill's GEMM (the float counterpart of
  * model/bitexact.py:121-125 matvec_ternary_rows, one weight pass for many rows): y[r] = W xhat_r
  * for n rows x_r of K floats (xhat = x, or x / rms(x) * norm_w with norm_w != NULL), on the matrix
- * cores. Ternary rows: xhat enters as five planes of base-32 digits with an exponent per 32 columns,
- * the trits as they are, and each 128-column sum is multiplied by the group's fp16 scale in float32
- * ((code - 1) * scale is what model/fastref.py:104-116's fp16 weight cache holds). Q8 rows are
- * decoded to that cache's fp16(q * scale) and xhat is split into fp16 hi and lo planes. Either way
- * each product is fp32-accurate. kind: TRX_KIND_TERNARY, TRX_KIND_TERNARY5 or TRX_KIND_Q8.
+ * cores. Ternary rows: xhat enters as five planes of digits with an exponent per 32 columns, the
+ * trits as they are, and each 128-column sum is multiplied by the group's fp16 scale in float32
+ * ((code - 1) * scale is what model/fastref.py:104-116's fp16 weight cache holds). A value of xhat
+ * is held to 2^-23 of its own leading power of two or 2^-25 of that of its 32 columns' largest,
+ * whichever is more; where the larger ones stand seven octaves or more above the others and four
+ * empty ones apart (and the others are seven, or fewer the further apart), to 2^-25 of the others'.
+ * Q8 rows are decoded to that cache's fp16(q * scale) and xhat is split into fp16 hi and lo planes
+ * (2^-23 of a value's leading power, 2^-25 of the row's scale). Sums are float32. kind:
+ * TRX_KIND_TERNARY, TRX_KIND_TERNARY5 or TRX_KIND_Q8.
  * Epilogues: TRX_EPI_STORE y [n][M]; TRX_EPI_RESID y [n][M] +=;
  * TRX_EPI_SWIGLU (rows [0,F) gate, [F,2F) up) y [n][M/2]. Inputs of any finite magnitude stay
  * finite (exponents per block, or per row for Q8: powers of two, exact). rows must be followed by 16

@@ -2,10 +2,10 @@
 
 The bound is derived: what the five digits leave of x is at most 2^-23 of its own leading power or 2^-25
 of its 32-column block's, whichever is more (2^-106 where the block lies below 2^-80, the smallest
-exponent): 2^-24 of the largest value plus two of the sums' half units cover both. A group's ten matrix instructions and the sums over the G groups round in float32 (2^-24 of the partial
-sums each, which the sum of |w x| bounds), and the output adds a few roundings (the RMSNorm's scale,
-the residual). Up to three values 2^7 or more above the rest of their block do not count as its
-largest.
+exponent): 2^-24 of the largest value plus two of the sums' half units cover both. A group's ten
+matrix instructions and the sums over the G groups round in float32 (2^-24 of the partial sums each,
+which the sum of |w x| bounds), and the output adds a few roundings (the RMSNorm's scale, the
+residual). Where values lie 2^7 or more above the rest of their block, the rest's own largest counts.
 """
 
 import ctypes
@@ -21,8 +21,10 @@ pytestmark = pytest.mark.gpu
 EPS = 1e-6
 
 
-def _matrix(kind, M, K, rng):
+def _matrix(kind, M, K, rng, silent=None):
     codes = rng.integers(0, 4 if kind == L.KIND_TERNARY else 3, (M, K)).astype(np.uint8)
+    if silent is not None:
+        codes[:, silent] = 1
     sc = rng.uniform(0.01, 0.05, (M, K // 128)).astype(np.float16)
     w = (codes.astype(np.float64) - 1).reshape(M, -1, 128) * sc.astype(np.float64)[:, :, None]
     return encode_rows(kind, K, sc, codes), w.reshape(M, K)
@@ -41,8 +43,8 @@ def _run(rows, kind, M, K, x, gain, epi, y0, work_offset=0):
     return yb.download(np.float32, n * cols).reshape(n, cols).astype(np.float64)
 
 
-def _check(kind, M, K, n, epi, norm, x, rng, work_offset=0, top=None):
-    rows, W = _matrix(kind, M, K, rng)
+def _check(kind, M, K, n, epi, norm, x, rng, work_offset=0, top=None, silent=None):
+    rows, W = _matrix(kind, M, K, rng, silent)
     gain = rng.uniform(0.8, 1.2, K).astype(np.float32) if norm else None
     y0 = rng.standard_normal((n, M)).astype(np.float32) if epi == _lib.EPI_RESID else None
     v = x.astype(np.float64)
@@ -187,3 +189,34 @@ def test_operands(kind, name, M, n):
     rms = [float(np.sqrt(np.mean(e * e))) for e in (err, _fp16_pair(x) - v)]
     print(f"{name} rms error {rms[0]:.2e}, of an fp16 pair {rms[1]:.2e}", flush=True)
     assert rms[0] <= rms[1]
+
+
+# A kernel's waves remember the groups that hold such blocks 64 apart: the last two shapes have more groups.
+LARGE = [(kind, big, count, M, K, n) for kind in (L.KIND_TERNARY5, L.KIND_TERNARY) for big in (3e2, 1e4, 1e18)
+         for count in (1, 3, 4, 8, 17, 24) for M, K, n in ((130, 1280, 41), (8190, 384, 1100))]
+LARGE += [(L.KIND_TERNARY5, 1e4, 6, 8192, 8448, 1100), (L.KIND_TERNARY, 1e4, 6, 34, 67584, 5)]
+
+
+@pytest.mark.parametrize("kind,big,count,M,K,n", LARGE)
+def test_large_values_leave_the_rest(kind, big, count, M, K, n):
+    """Any number of values far above the rest of their block, in some blocks of every row: outputs whose weights on
+    them are 0 are as exact as if they were small (the bound takes the rest's largest value)."""
+    rng = np.random.default_rng(count + M)
+    x = rng.standard_normal((n, K))
+    cols = np.zeros(K, bool)
+    for b in list(rng.permutation(K // 32 - 1)[:4]) + [K // 32 - 1]:
+        # From the block's second column on: the blocks of a trit5 half 1 end one column later.
+        cols[32 * b + 1 + rng.permutation(31)[:count]] = True
+    rest = np.abs(x * ~cols).reshape(n, K // 128, 128).max(axis=2).repeat(128, axis=1)
+    x[:, cols] = rng.choice([-1, 1], (n, cols.sum())) * big * rng.uniform(1, 1.9, (n, cols.sum()))
+    _check(kind, M, K, n, _lib.EPI_STORE, False, x.astype(np.float32), rng, top=rest, silent=cols)
+
+
+def test_few_values_among_zeros():
+    rng = np.random.default_rng(11)
+    x = np.zeros((40, 512), np.float32)
+    x[:, 5], x[:, 9], x[:, 20] = 1e6, 1.5, -0.7
+    x[:, 300] = 0.9
+    silent = np.zeros(512, bool)
+    silent[5] = True
+    _check(L.KIND_TERNARY5, 200, 512, 40, _lib.EPI_STORE, False, x, rng, top=np.ones(x.shape), silent=silent)

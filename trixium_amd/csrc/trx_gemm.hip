@@ -3,7 +3,7 @@
 // x enters as five planes of digits in fp6 (E2M3), W's trits as fp4 (E2M1), so that the products run on
 // v_mfma_scale_f32_32x32x64_f8f6f4 at its fp6/fp4 rate, four times fp16's:
 //   x = 2^u (d0 + d1/2^5 + d2/2^10 + d3/2^15 + d4/2^21), every digit a whole number of the format's eighths
-// with one exponent u per position and 32 columns (the largest |x| in [16, 32) * 2^u, but see Lone). E2M3 holds
+// with one exponent u per position and 32 columns (the largest |x| in [16, 32) * 2^u). E2M3 holds
 // whole eighths up to 2, every second one up to 4 and every fourth up to 7.5, and E2M1 holds -1, 0, 1 (and 2,
 // the 2-bit code 3); the plane's power of two is the instruction's block scale, and its fp32 accumulation of
 // such products is exact while a sum fits 24 bits. A value of the block's highest octave leaves up to four
@@ -36,17 +36,31 @@ typedef float f32x32_t __attribute__((ext_vector_type(32)));
 // 63, step s its 32 from 32 s on (trit5: half 1 takes columns 65 .. 127 and then 64, whose code
 // shares a byte with half 0's). A position tile's step is 256 P bytes for its P <= 32 positions:
 // eight runs [h][j] of 16-byte pieces that hold a lane's 32 dwords in order, six of each plane (the
-// lowest digit's first), then the block's scales and the fp32 sum of the 32 columns' x^2. Four bytes a column in all, read by 16-byte loads only (per byte, the
-// vector cache is a quarter slower on 8- and 12-byte ones).
+// lowest digit's first), then the block's scales and the fp32 sum of the 32 columns' x^2. Four bytes a
+// column in all, read by 16-byte loads only (per byte, the vector cache is a quarter slower on 8- and
+// 12-byte ones).
 constexpr int kPlanes = 5;
 constexpr int kUMin = -85;             // smallest u: below it values lose bits under 2^-106
-constexpr int kApart = 7;
 // The block scales hold the planes 2^16 down and the weights' scales 2^16 up, so that no group's sum
 // of finite values overflows.
 constexpr int kScaleByte = 109 - 16;
 // Plane c's power of two above plane 0's.
 constexpr uint32_t plane_up(int c) { return c ? 5 * c + 1 : 0; }
 constexpr float kScaleUp = 65536.f;
+// Wide blocks. Five digits hold what lies far below a block's largest value to few bits of its own, which
+// shows where a row's weights on the larger values are 0 (a model's massive channels). A block is wide, and its
+// values take part one by one (Wide), if some lie seven octaves or more below the largest and behind at least
+// four empty octaves, the empty ones times these values 28 or more (four octaves and seven values, seven and
+// four, fourteen and two), or if twelve, an octave counted for two at most, lie ten octaves or more below.
+// Values 128 times their neighbours do that; of the blocks of normal, product and SwiGLU inputs, also with
+// channels 20 times larger, fewer than 1e-6 do (their smallest values lie apart by chance).
+// A wide block holds its values in 30 bits each, the sign, 6 bits of exponent and all of the fraction: value e in
+// the low bits of dword e, the last two in the 30 dwords' high pairs of bits. Exponents 32 to 62 count from the
+// largest value's (62) down, 1 to 31 from the largest of those below (31); 0 is 0 or less than 2^-31 of that. In
+// place of the scales stand a bit that marks the block, the octaves down to the others, the two largest values'
+// exponents and scale 0 (the digits' part of the products, of these bits, drowns: below 2^-58 of the
+// largest value). Blocks below 2^-40 stay as they are: their digits leave out 2^-65.
+constexpr int kWideTop = 127 - 40;
 
 // A lane packs one position's 32 columns with the hardware's fp6 conversions (digit by digit in floats it
 // would take ~35 vector operations a column). Bound by memory on long prompts: 2048 x 12288 in 40 us,
@@ -106,62 +120,94 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
     top = max(top, max(__float_as_uint(a[i]) & 0x7FFFFFFFu, __float_as_uint(b[i]) & 0x7FFFFFFFu));
   }
   const bool finite = top < 0x7F800000u;
-  // One to three values 2^kApart or more above the rest (see Lone values below): the block's exponent is
-  // the rest's, and they go in 2^-apart times. u from an exponent field E: E - 131.
-  const uint32_t high = top > ((uint32_t)kApart << 23) ? top - ((uint32_t)kApart << 23) : 0;
-  uint32_t rest = 0;
-  int count = 0;
+  // The octaves, from the largest value's (bit 0) down, that hold a value and those that hold more; the last
+  // bit stands for all from there on, and 0.
+  const int et = (int)(top >> 23);
+  uint32_t seen = 0, more = 0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t ma = __float_as_uint(a[i]) & 0x7FFFFFFFu, mb = __float_as_uint(b[i]) & 0x7FFFFFFFu;
-    count += (ma >= high) + (mb >= high);
-    rest = max(rest, max(ma >= high ? 0u : ma, mb >= high ? 0u : mb));
+  for (int i = 0; i < 32; ++i) {
+    const int E = (int)(__float_as_uint(i & 1 ? b[i >> 1] : a[i >> 1]) >> 23 & 0xFFu);
+    const uint32_t bit = 1u << (max(E, et - 31) & 31);
+    more |= seen & bit;
+    seen |= bit;
   }
-  int u = max((int)(top >> 23) - 131, kUMin), apart = 0;
-  uint32_t where = 0;
-  if (finite && rest != 0 && count <= 3) {
-    const int un = max((int)(rest >> 23) - 131, kUMin);
-    apart = u - un;
-    u = un;
-    auto lone = [&](float x, int e) {
-      if ((__float_as_uint(x) & 0x7FFFFFFFu) < high) return x;
-      where = where << 5 | (uint32_t)e;
-      return ldexpf(x, -apart);
-    };
+  auto from_top = [&](uint32_t v) { return __builtin_bitreverse32(__builtin_amdgcn_alignbit(v, v, et + 1)); };
+  seen = from_top(seen);
+  more = from_top(more);
+  int n = 0;                                          // the last's values without the zeros
+  if ((int)seen < 0) {
+    asm volatile("" : "+v"(a), "+v"(b));              // or the 32 exponents stay in registers from above
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      a[i] = lone(a[i], 2 * i);
-      b[i] = lone(b[i], 2 * i + 1);
+    for (int i = 0; i < 32; ++i) {
+      const int E = (int)(__float_as_uint(i & 1 ? b[i >> 1] : a[i >> 1]) >> 23 & 0xFFu);
+      n += E > 0 && E <= et - 31;
     }
-    for (; count < 3; ++count) where = where << 5 | (where & 31u);
+    seen = (seen & 0x7FFFFFFFu) | (n > 0 ? 0x80000000u : 0u);
   }
+  auto count = [&](uint32_t mask) { return __popc(seen & mask & 0x7FFFFFFFu) + __popc(more & mask & 0x7FFFFFFFu) + n; };
+  const uint32_t z = ~seen & ~seen >> 1 & ~seen >> 2 & ~seen >> 3 & 0x0FFFFFFFu;    // four empty ones from here
+  const int from = z ? __builtin_ctz(z) : 0;
+  const uint32_t low = z ? ~0u << (from + 3) << 1 : 0u;
+  const int first = __builtin_ctz(seen & low | 0x80000000u), gap = first - from;
+  int others = low ? count(low) : 0;
+  if (first >= 7 && others > 1 && others * gap < 28) {               // how many they are
+    asm volatile("" : "+v"(a), "+v"(b));
+    others = 0;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const int E = (int)(__float_as_uint(i & 1 ? b[i >> 1] : a[i >> 1]) >> 23 & 0xFFu);
+      others += E > 0 && E <= et - first;
+    }
+  }
+  const bool apart = first >= 7 && others * gap >= 28;
+  const bool wide = finite && et >= kWideTop && (apart || count(~0u << 10) >= 12);
   uint8_t* out = p.xp + (size_t)32 * pt * p.K * 4 + (size_t)st * 256 * P;
   uint4* o = (uint4*)out + h * P + j;
   uint32_t dw[32];
+  if (!wide) {
+    const int u = max(et - 131, kUMin);               // 2^(E - 127 - 4) from an exponent field E
 #pragma unroll
-  for (int d = 0; d < kPlanes; ++d) {
-    const int c = kPlanes - 1 - d;
-    const float sc = __uint_as_float((uint32_t)(u + 3 - 21 + (int)plane_up(c) + 127) << 23);
-    const u32x6_t q = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, sc);
-    // The sources stay live past the conversion: it reads them while it writes its result, and the
-    // compiler may otherwise give both the same registers.
-    asm volatile("" ::"v"(a), "v"(b));
-    if (d + 1 < kPlanes) {
-      const f32x32_t back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
-      asm volatile("" ::"v"(q));
+    for (int d = 0; d < kPlanes; ++d) {
+      const int c = kPlanes - 1 - d;
+      const float sc = __uint_as_float((uint32_t)(u + 3 - 21 + (int)plane_up(c) + 127) << 23);
+      const u32x6_t q = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, sc);
+      // The sources stay live past the conversion: it reads them while it writes its result, and the
+      // compiler may otherwise give both the same registers.
+      asm volatile("" ::"v"(a), "v"(b));
+      if (d + 1 < kPlanes) {
+        const f32x32_t back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(q, sc);
+        asm volatile("" ::"v"(q));
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        a[i] -= back[2 * i];
-        b[i] -= back[2 * i + 1];
+        for (int i = 0; i < 16; ++i) {
+          a[i] -= back[2 * i];
+          b[i] -= back[2 * i + 1];
+        }
       }
-    }
 #pragma unroll
-    for (int i = 0; i < 6; ++i) dw[6 * c + i] = q[i];
+      for (int i = 0; i < 6; ++i) dw[6 * c + i] = q[i];
+    }
+    // Byte 0: the block scale of the lowest plane (plane c's is plane_up(c) above); 0xFF, the format's NaN, where
+    // a value is not finite.
+    dw[30] = finite ? (uint32_t)(u + kScaleByte) : 0xFFu;
+  } else {
+    uint32_t next = 0;                                // the largest 31 octaves down or more
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const uint32_t m = __float_as_uint(i & 1 ? b[i >> 1] : a[i >> 1]) & 0x7FFFFFFFu;
+      next = max(next, (int)(m >> 23) <= et - 31 ? m : 0u);
+    }
+    const uint32_t eb = next >> 23;
+    auto code = [&](float x) {
+      const uint32_t v = __float_as_uint(x), m = v & 0x7FFFFFFFu, E = m >> 23;
+      const uint32_t at = (int)E > et - 31 ? E + 62 - (uint32_t)et : E && E + 31 > eb ? E + 31 - eb : 0u;
+      return (at ? at << 23 | (m & 0x7FFFFFu) : 0u) | (v >> 31) << 29;
+    };
+    const uint32_t c30 = code(a[15]), c31 = code(b[15]);
+#pragma unroll
+    for (int i = 0; i < 30; ++i)
+      dw[i] = code(i & 1 ? b[i >> 1] : a[i >> 1]) | (i < 15 ? c30 >> (2 * i) : c31 >> (2 * (i - 15))) << 30;
+    dw[30] = 0x80000000u | (apart ? (uint32_t)first : 31u) << 24 | eb << 16 | (uint32_t)et << 8;
   }
-  // Byte 0: the block scale of the lowest plane (plane c's is plane_up(c) above); 0xFF, the format's NaN, where a
-  // value is not finite. Byte 1: the lone values' shift; then their three places and bit 31.
-  dw[30] = !finite ? 0xFFu
-                   : (uint32_t)(u + kScaleByte) | (apart > 0 ? (uint32_t)apart << 8 | where << 16 | 0x80000000u : 0u);
   dw[31] = __float_as_uint(ss);
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[2 * P * i] = make_uint4(dw[4 * i], dw[4 * i + 1], dw[4 * i + 2], dw[4 * i + 3]);
@@ -278,64 +324,61 @@ __device__ __forceinline__ int tile_row(int tile, int j, int M) {
   return min(32 * tile + j, M);
 }
 
-// Lone values. A block's values share an exponent, so a few far above the rest would cost the rest their
-// low bits (a model's massive channels do that; the result's norm would not show it, outputs whose
-// weight there is 0 would). planes_kernel stores such a value v as v' = 2^-apart v at the others'
-// scale. Tiles that met one (a bit of the scales) go over K once more and add v - v' for the steps
-// that hold one: the planes masked to the values' places, once at their scale and once negated at the
-// block's.
-template <int C>
-__device__ __forceinline__ f32x16_t mx_lone(const Planes& q, const i32x4_t& w, f32x16_t acc) {
-  const uint32_t s = q.scales();
-  const bool on = (int)s < 0;
-  const i32x8_t x = q.get<C>();
-  i32x8_t A = {}, N = {};
+// A step's wide blocks, digit by digit, from the highest on until less is left than 2^-25 of the others' leading
+// power (where they lie 31 octaves down or are no cluster of their own: nothing); a lane without one gives zeros.
+struct Wide {
+  f32x16_t a, b;
+  int e, stop;                         // exponent fields: the next digit's unit, the least that takes one
+  __device__ __forceinline__ void init(const Planes& q) {
+    const uint32_t s = q.scales();
+    const bool on = (int)s < 0;
+    const uint32_t et = on ? s >> 8 & 0xFFu : 127u, eb = on ? s >> 16 & 0xFFu : 0u;
+    uint32_t dw[30], c30 = 0, c31 = 0;
 #pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    uint32_t mask = 0, sign = 0;                      // a place's six bits, the last its sign
+    for (int i = 0; i < 30; ++i) dw[i] = on ? (uint32_t)(i < 12 ? q.c01[i % 12] : i < 24 ? q.c23[i % 12] : q.c4[i % 6]) : 0u;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int sh = 6 * (int)(s >> (16 + 5 * k) & 31u) - 32 * i;
-      if (on && sh > -6 && sh < 32) mask |= sh >= 0 ? 0x3Fu << sh : 0x3Fu >> -sh;
-      if (on && sh >= -5 && sh < 27) sign |= 1u << (sh + 5);
+    for (int i = 0; i < 15; ++i) {
+      c30 |= dw[i] >> 30 << (2 * i);
+      c31 |= dw[15 + i] >> 30 << (2 * i);
     }
-    A[i] = (int)((uint32_t)x[i] & mask);
-    N[i] = A[i] ^ (int)sign;
-  }
-  const i32x8_t B = {w[0], w[1], w[2], w[3], 0, 0, 0, 0};
-  const uint32_t s0 = (s & 0xFFu) + plane_up(C);
-  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(N, B, acc, 2, 4, 0, (int)s0, 0, 0x7F7F7F7F);
-  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, acc, 2, 4, 0, (int)(s0 + (on ? s >> 8 & 0xFFu : 0u)), 0,
-                                                          0x7F7F7F7F);
-}
-__device__ __forceinline__ void mx_lone_step(const Planes& q, const i32x4_t& w, f32x16_t& t) {
-  t = mx_lone<0>(q, w, t);
-  t = mx_lone<1>(q, w, t);
-  t = mx_lone<2>(q, w, t);
-  t = mx_lone<3>(q, w, t);
-  t = mx_lone<4>(q, w, t);
-}
-// acc += the lone values of groups g0 .. g1 - 1 times one tile of weights.
-template <int KIND, int EPI>
-__device__ __forceinline__ void add_lone(const GemmParams& p, const PlaneReader& pl, int tile, const uint32_t* lut, int g0,
-                                         int g1, f32x16_t& acc) {
-  const int lane = threadIdx.x & 63;
-  RowReader<KIND> row;
-  row.init(p, tile_row<EPI>(tile, lane & 31, p.M), lane >> 5);
-  for (int g = g0; g < g1; ++g) {
-    const uint32_t s = (uint32_t)pl.piece(pl.base(2 * g), 7)[2] | (uint32_t)pl.piece(pl.base(2 * g + 1), 7)[2];
-    if (!__any((int)s < 0)) continue;
-    Codes codes;
-    row.load(codes, g);
-    uint32_t D[8];
-    row.decode(codes, g, lut, D);
-    f32x16_t t = {};
-    mx_lone_step(pl.load(2 * g), i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]}, t);
-    mx_lone_step(pl.load(2 * g + 1), i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]}, t);
-    const float sc = row_scale<KIND>(row, codes);
+    auto value = [&](uint32_t c) {
+      const uint32_t m = c & 0x1FFFFFFFu, from = m >= 32u << 23 ? et - 62u : eb - 31u;
+      return __uint_as_float((m ? m + (from << 23) : 0u) | (c & 0x20000000u) << 2);
+    };
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = fmaf(t[e], sc, acc[e]);
+    for (int i = 0; i < 16; ++i) {
+      a[i] = value(i < 15 ? dw[2 * i] : c30);
+      b[i] = value(i < 15 ? dw[2 * i + 1] : c31);
+    }
+    e = (int)et - 1;
+    stop = max(on && (s >> 24 & 31u) < 31u ? (int)et - (int)(s >> 24 & 31u) - 25 : 0, 20);
   }
+  // The next digit and its block scale; whether any lane has more.
+  __device__ __forceinline__ bool next(u32x6_t& c, int& scale) {
+    const float sc = __uint_as_float((uint32_t)e << 23);
+    scale = e - 16;
+    c = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(a, b, sc);
+    asm volatile("" ::"v"(a), "v"(b));                // see planes_kernel
+    const f32x32_t back = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(c, sc);
+    asm volatile("" ::"v"(c));
+    float left = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      a[i] -= back[2 * i];
+      b[i] -= back[2 * i + 1];
+      left = fmaxf(fmaxf(left, fabsf(a[i])), fabsf(b[i]));
+    }
+    // Down to the largest that is left, past empty octaves; below 2^-107 nothing is.
+    const int el = (int)(__float_as_uint(left) >> 23);
+    const bool more = el >= stop;
+    e = more ? min(e - 5, el - 1) : 17;
+    return __any(more);
+  }
+};
+__device__ __forceinline__ f32x16_t mx_digits(const u32x6_t& c, int scale, const i32x4_t& w, const f32x16_t& acc) {
+  const i32x8_t A = {(int)c[0], (int)c[1], (int)c[2], (int)c[3], (int)c[4], (int)c[5], 0, 0};
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, i32x8_t{w[0], w[1], w[2], w[3], 0, 0, 0, 0}, acc, 2, 4, 0, scale,
+                                                         0, 0x7F7F7F7F);
 }
 
 // Block b of nx weight tiles x ny position tiles. Blocks go to the 8 XCDs in turn; each XCD takes
@@ -386,6 +429,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
   __shared__ __align__(16) i32x4_t bs[2][NT][2][64];
   __shared__ float wsc[2][32 * NT];
   __shared__ float rsx[128];
+  __shared__ unsigned long long wide_of[4];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5, j = lane & 31;
   int bx, by;
   tile_of_block(blockIdx.x, p.nx, p.ny, bx, by);
@@ -419,7 +463,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
   f32x16_t acc[NT] = {}, t[2][2] = {};
   i32x4_t wt[2][2][2];                                // [pair's parity][step][tile]
   float sc[2][2] = {}, ss = 0.f;
-  int lone = 0;
+  unsigned long long wide = 0;                        // groups with wide blocks, 64 apart
   wt[0][0][0] = bs[0][0][0][lane];
   wt[0][0][1] = bs[0][1][0][lane];
   wt[0][1][0] = bs[0][0][1][lane];
@@ -439,7 +483,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
     t[T][1] = mx<C % 5>(q, wt[T][ST][1], C ? t[T][1] : zero);
     asm volatile("" : "+v"(t[T][0]), "+v"(t[T][1]) : : "memory");
     if constexpr (S == 4 || S == 9) {
-      lone |= __any((int)q.scales() < 0);
+      wide |= (unsigned long long)(__any((int)q.scales() < 0) ? 1u : 0u) << (g & 63);
       ss += q.ss();
       asm volatile("" : "+a"(ss));
     }
@@ -501,9 +545,70 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
   for (int k = 0; k < 2; ++k)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[NT - 2 + k][e] = fmaf(t[1][k][e], sc[1][k], acc[NT - 2 + k][e]);
-  if (lone) {
+
+  // The groups in which any wave met a wide block once more: the weights decoded by all as above, the products
+  // by the waves that hold one, a digit of x for all tiles at a time under the next digit's conversion. About
+  // 6 us a group and block: 24576 x 4096, 2048 positions, takes 514 us without wide blocks, 549, 650 and 1079
+  // with one, four and sixteen channels 1000 times the others at every position (a pass for each tile, its
+  // loads one by one: 843, 1144 and 2469; two fp16 planes, with or without: 750).
+  if (!live) wide = 0;
+  if (lane == 0) wide_of[w] = wide;
+  __syncthreads();
+  const unsigned long long some = wide_of[0] | wide_of[1] | wide_of[2] | wide_of[3];
+  if (some) {
+    // The sums leave the vector registers for this, or the main loop's own registers are spilt to make room.
 #pragma unroll
-    for (int b = 0; b < NT; ++b) add_lone<KIND, EPI>(p, pl, NT * bx + b, lut, 0, G, acc[b]);
+    for (int b = 0; b < NT; ++b) asm volatile("" : "+a"(acc[b]));
+    auto next_wide = [&](int g) {
+      while (g < G && !(some >> (g & 63) & 1)) ++g;
+      return g;
+    };
+    int g = next_wide(0);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) row[d].load(codes[d], min(g, G - 1));
+    while (g < G) {
+      const int gn = next_wide(g + 1);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        uint32_t D[8];
+        row[d].decode(codes[d], g, lut, D);
+        bs[0][4 * d + w][0][lane] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
+        bs[0][4 * d + w][1][lane] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
+        wsc[0][32 * (4 * d + w) + j] = row_scale<KIND>(row[d], codes[d]);
+        row[d].load(codes[d], min(gn, G - 1));
+      }
+      __syncthreads();
+      if (wide >> (g & 63) & 1) {
+        f32x16_t s[NT] = {};
+#pragma nounroll
+        for (int st = 0; st < 2; ++st) {
+          const Planes q = pl.load(2 * g + st);
+          if (!__any((int)q.scales() < 0)) continue;
+          i32x4_t wd[NT];
+#pragma unroll
+          for (int b = 0; b < NT; ++b) wd[b] = bs[0][b][st][lane];
+          Wide x;
+          x.init(q);
+          bool more = true;
+#pragma nounroll
+          while (more) {
+            u32x6_t c;
+            int scale;
+            more = x.next(c, scale);
+#pragma unroll
+            for (int b = 0; b < NT; ++b) s[b] = mx_digits(c, scale, wd[b], s[b]);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+          const float v = wsc[0][32 * b + j];
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[b][e] = fmaf(s[b][e], v, acc[b][e]);
+        }
+      }
+      __syncthreads();
+      g = gn;
+    }
   }
 
   // Accumulator e of lane l holds position i = 8 (e / 4) + 4 (l / 32) + e % 4, weight row l % 32.
@@ -572,7 +677,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
   __syncthreads();
   f32x16_t acc[NB] = {};
   float ss = 0.f;
-  uint32_t lone = 0;
+  unsigned long long wide = 0;                        // groups with wide blocks, 64 apart
   for (int g = g0; g < g1; ++g) {
     i32x4_t b0[NB], b1[NB];
     float sc[NB];
@@ -587,7 +692,7 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
       asm volatile("" : "+v"(b0[b]), "+v"(b1[b]) : : "memory");
       row[b].load(codes[b], gn);
     }
-    lone |= q0.scales() | q1.scales();
+    wide |= (unsigned long long)(__any((int)(q0.scales() | q1.scales()) < 0) ? 1u : 0u) << ((g - g0) & 63);
     f32x16_t t[NB];
     ss += q0.ss();
     mx_step<true, NB>(q0, b0, t);
@@ -603,9 +708,46 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[b][e] = fmaf(t[b][e], sc[b], acc[b][e]);
   }
-  if (__any((int)lone < 0)) {
+  if (wide) {
+    constexpr int TB = NB < 2 ? 1 : 2;                // tiles at a time (registers)
+    for (int g = g0; g < g1; ++g) {
+      if (!(wide >> ((g - g0) & 63) & 1)) continue;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) add_lone<KIND, EPI>(p, pl, NB * bx + b, sm, g0, g1, acc[b]);
+      for (int t0 = 0; t0 < NB; t0 += TB) {
+        i32x4_t b0[TB], b1[TB];
+        float sc[TB];
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+          row[t0 + b].load(codes[b], g);
+          uint32_t D[8];
+          row[t0 + b].decode(codes[b], g, sm, D);
+          b0[b] = i32x4_t{(int)D[0], (int)D[1], (int)D[2], (int)D[3]};
+          b1[b] = i32x4_t{(int)D[4], (int)D[5], (int)D[6], (int)D[7]};
+          sc[b] = row_scale<KIND>(row[t0 + b], codes[b]);
+        }
+        f32x16_t s[TB] = {};
+#pragma nounroll
+        for (int st = 0; st < 2; ++st) {
+          const Planes q = pl.load(2 * g + st);
+          if (!__any((int)q.scales() < 0)) continue;
+          Wide x;
+          x.init(q);
+          bool more = true;
+#pragma nounroll
+          while (more) {
+            u32x6_t c;
+            int scale;
+            more = x.next(c, scale);
+#pragma unroll
+            for (int b = 0; b < TB; ++b) s[b] = mx_digits(c, scale, st ? b1[b] : b0[b], s[b]);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[t0 + b][e] = fmaf(s[b][e], sc[b], acc[t0 + b][e]);
+      }
+    }
   }
   ss += __shfl_xor(ss, 32, 64);
   if (h == 0) ssx[w][j] = ss;
