@@ -350,12 +350,15 @@ static int ensure_packed(Model& m) {
 static int dalloc(Model& m, void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes + 256);
   if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
     set_error("device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? TRX_E_NOMEM : TRX_E_HIP;
   }
   m.allocs.push_back(*p);
   m.dev_bytes += bytes;
   TRX_HIP(hipMemset(*p, 0, bytes + 256));
+  TRX_HIP(hipStreamSynchronize(nullptr));          // the model's stream does not wait for that one
   return TRX_OK;
 }
 
@@ -962,8 +965,14 @@ static int pf_alloc(Model& m, int R) {
   }
   int cap = 64;
   while (cap < R) cap *= 2;
-  for (auto& b : bufs)
-    if (b.second && (rc = dalloc(m, b.first, b.second * (size_t)cap))) return rc;
+  for (auto& b : bufs) {
+    if (!b.second || !(rc = dalloc(m, b.first, b.second * (size_t)cap))) continue;
+    for (auto& f : bufs) {                           // none of them, then
+      (void)dfree(m, *f.first, f.second * (size_t)cap);
+      *f.first = nullptr;
+    }
+    return rc;
+  }
   m.pf_rows = cap;
   return TRX_OK;
 }
@@ -1609,10 +1618,8 @@ TRX_API int trx_model_score(trx_model* h, const int32_t* tokens, int n, float* n
   const trx_model_config& c = m.cfg;
   TRX_CHECK(n <= c.max_ctx, TRX_E_STATE, "trx_model_score: %d tokens exceed max_ctx %d", n, c.max_ctx);
   int rc;
-  if (!m.nll) {
-    if ((rc = dalloc(m, (void**)&m.nll, (size_t)c.max_ctx * 4))) return rc;
-    if ((rc = dalloc(m, (void**)&m.hid_rows, (size_t)c.max_ctx * c.n_embd * 4))) return rc;
-  }
+  if (!m.nll && (rc = dalloc(m, (void**)&m.nll, (size_t)c.max_ctx * 4))) return rc;
+  if (!m.hid_rows && (rc = dalloc(m, (void**)&m.hid_rows, (size_t)c.max_ctx * c.n_embd * 4))) return rc;
   if ((rc = trx_model_reset(h))) return rc;
   if ((rc = trx_model_set_prompt(h, tokens, n, 0))) return rc;
   // All positions but the last through the batched prefill and a GEMM of the head, unless the sampler
@@ -1645,10 +1652,8 @@ TRX_API int trx_model_project_head(trx_model* h, const float* hidden, int n, flo
   int rc;
   if ((rc = check_loaded(m))) return rc;
   if ((rc = ensure_packed(m))) return rc;
-  if (!m.proj_x) {
-    if ((rc = dalloc(m, (void**)&m.proj_x, (size_t)c.n_embd * 4))) return rc;
-    if ((rc = dalloc(m, (void**)&m.proj_y, (size_t)c.vocab * 4))) return rc;
-  }
+  if (!m.proj_x && (rc = dalloc(m, (void**)&m.proj_x, (size_t)c.n_embd * 4))) return rc;
+  if (!m.proj_y && (rc = dalloc(m, (void**)&m.proj_y, (size_t)c.vocab * 4))) return rc;
   const int head_role = c.head_tied ? TRX_ROLE_TOK_EMB : TRX_ROLE_LM_HEAD;
   const int head_kind = c.head_tied ? c.emb_kind : c.head_kind;
   for (int i = 0; i < n; ++i) {
