@@ -386,8 +386,11 @@ int trx_model_read(trx_model* m, int what, void* host, size_t bytes);
  * the model): nll[i] = logsumexp(logits_i) - logits_i[tokens[i + 1]] for i < n - 1 (host float32,
  * may be NULL), and the final normed hidden states hidden[n][n_embd] (host, may be NULL,
  * fastref.py:244-258 hidden). Synchronous; every position but the last goes through the batched
- * prefill and a product with the LM head over 128 positions at a time (with the sampler on, which
- * draws at every position, or an fp16 head, one position per forward). */
+ * prefill, up to 1024 at a time, and a product with the LM head over 128 at a time. Its buffers
+ * (those of trx_model_prefill and 128 * vocab floats) stay until the model is destroyed. With the
+ * sampler on, which draws at every position, with a head in another format than the layers or a
+ * shape that the batched kernels do not take, or without room for the buffers: one position per
+ * forward. */
 int trx_model_score(trx_model* m, const int32_t* tokens, int n, float* nll, float* hidden);
 /* The LM head applied to n given hidden states (host float32 [n][n_embd] -> [n][vocab]):
  * model/fastref.py:260-261 logits (the rotation of a rotated model included, no norm).

@@ -1,12 +1,14 @@
 """Decoder.score over the batched prefill (model/fastref.py:244-273), for models with a ternary LM head:
 NLLs and hidden states against one-position forwards, and what the call leaves behind."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
-from trixium_amd import configs as C
+from trixium_amd import _lib, configs as C, layout as L
 from trixium_amd import synth
-from trixium_amd.model import Decoder
+from trixium_amd.model import Decoder, make_config
 
 pytestmark = pytest.mark.gpu
 
@@ -44,4 +46,19 @@ def test_score_matches_forwards(mc, rot, n):
     dec.set_sampling(0.8, 0.9, 1.1, 7)
     nll1, hid1 = dec.score(toks)
     assert _rel_err(hid1, hid) <= 2e-3 and np.all(np.abs(nll1 - want) <= 2e-3 * max(1.0, np.max(np.abs(want), initial=0)))
+    dec.close()
+
+
+def test_kv_pin_holds_through_a_score():
+    """A pin holds for the next reset, which is the score's own, also where the model's head (here in the other
+    code format) is one that the batched pass does not take."""
+    mc = C.TINY.replace(tie_embeddings=False)
+    dec = Decoder(mc, make_config(mc, L.KIND_TERNARY5, L.KIND_TERNARY, False, 1, L.KIND_TERNARY5))
+    ranges = np.array([0.01, 0.04, 0.8, 0.4], np.float32)
+    _lib.call("trx_model_synthesize", dec._h, 3, ranges.ctypes.data_as(ctypes.POINTER(ctypes.c_float)))
+    toks = synth.random_prompt(mc, 20, 1)
+    for pin in (9, 12):
+        dec.set_kv_ring(1, pin)
+        dec.score(toks)
+        assert dec.kv_pin == pin
     dec.close()

@@ -32,6 +32,7 @@ struct Tensor {
 // sampler's repetition window (the last 64 tokens, firmware/infer.c:385-488).
 constexpr int kKvSinks = 4;
 constexpr int kScoreRows = 128;        // positions per LM head product when scoring
+constexpr int kScoreChunk = 1024;      // and per batched prefill
 constexpr int kPfPartRow = 16 * 128;   // floats of K-part sums per prefill row
 constexpr int kSmpWindow = 64;
 
@@ -1568,6 +1569,30 @@ TRX_API int trx_model_generate(trx_model* h, const int32_t* prompt, int n_prompt
   return check_err(m);
 }
 
+// Whether every kernel of score_batched takes the model: the batched prefill's, and the GEMM for the head
+// (its input's planes are in the order of the layers' code format).
+static bool score_takes(const Model& m) {
+  const trx_model_config& c = m.cfg;
+  const int hd = c.head_dim, rope_n = c.rope_dims ? c.rope_dims : hd;
+  const int nq = c.dn_num_k_heads * c.dn_k_head_dim, nvh = c.dn_num_v_heads * c.dn_v_head_dim;
+  const long long widest = std::max<long long>({c.vocab, 2ll * c.ffn_dim, 2ll * c.n_head * hd + 2ll * c.n_kv_head * hd,
+                                                2ll * nq + 2ll * nvh});
+  const int kmax = std::max({c.n_embd, c.ffn_dim, c.n_head * hd, nvh});
+  return (c.head_tied ? c.emb_kind : c.head_kind) == c.weight_kind &&
+         widest * row_bytes_of(c.weight_kind, kmax) < (1ll << 32) && (size_t)kScoreChunk * kmax * 2 < (1ull << 32) &&
+         (!m.n_attn || attn_rows_take(c.n_head, c.n_kv_head, hd, rope_n, c.max_ctx)) &&
+         (!m.n_dn || dn_rows_take(2 * nq + nvh, c.dn_conv_kernel, c.dn_num_v_heads, c.dn_num_k_heads, c.dn_k_head_dim,
+                                  c.dn_v_head_dim));
+}
+
+// The buffers of score_batched over n positions.
+static int score_alloc(Model& m, int n, bool want_nll) {
+  int rc;
+  if ((rc = pf_alloc(m, std::min(n, kScoreChunk)))) return rc;
+  if (want_nll && !m.score_logits) return dalloc(m, (void**)&m.score_logits, (size_t)kScoreRows * m.cfg.vocab * 4);
+  return TRX_OK;
+}
+
 // Positions 0 .. n - 1 of a teacher-forced sequence (fed, the model reset): the batched prefill, then
 // the normed hidden states and, with want_nll, the head over kScoreRows positions at a time and
 // their next tokens' NLLs. One position per forward reads every weight of the model for it (192
@@ -1575,13 +1600,8 @@ TRX_API int trx_model_generate(trx_model* h, const int32_t* prompt, int n_prompt
 static int score_batched(Model& m, int n, bool want_nll) {
   const trx_model_config& c = m.cfg;
   const int head_role = c.head_tied ? TRX_ROLE_TOK_EMB : TRX_ROLE_LM_HEAD;
-  const int head_kind = c.head_tied ? c.emb_kind : c.head_kind;
-  if (head_kind != c.weight_kind) return TRX_E_INVALID;         // the planes are in that kind's order
+  const int chunk = std::min(n, kScoreChunk), E = c.n_embd;
   int rc;
-  if ((rc = check_loaded(m))) return rc;
-  const int chunk = std::min(n, 1024), E = c.n_embd;
-  if ((rc = pf_alloc(m, chunk))) return rc;
-  if (want_nll && !m.score_logits && (rc = dalloc(m, (void**)&m.score_logits, (size_t)kScoreRows * c.vocab * 4))) return rc;
   for (int p0 = 0; p0 < n; p0 += chunk) {
     const int R = std::min(chunk, n - p0);
     if ((rc = run_prefill(m, p0, R, m.stream))) return rc;
@@ -1596,7 +1616,7 @@ static int score_batched(Model& m, int n, bool want_nll) {
     for (int r0 = 0; want_nll && r0 < R; r0 += kScoreRows) {
       const int rows = std::min(kScoreRows, R - r0);
       if ((rc = pf_prep(m, m.pf_x + (size_t)r0 * E, E, E, rows, sp.out_norm, m.stream))) return rc;
-      if ((rc = pf_gemm(m, head_role, 0, head_kind, c.vocab, E, rows, GM_STORE, m.score_logits, c.vocab, m.stream))) return rc;
+      if ((rc = pf_gemm(m, head_role, 0, c.weight_kind, c.vocab, E, rows, GM_STORE, m.score_logits, c.vocab, m.stream))) return rc;
       ScoreRowsParams lp = {};
       lp.n = E;
       lp.R = rows;
@@ -1622,16 +1642,19 @@ TRX_API int trx_model_score(trx_model* h, const int32_t* tokens, int n, float* n
   if (!m.hid_rows && (rc = dalloc(m, (void**)&m.hid_rows, (size_t)c.max_ctx * c.n_embd * 4))) return rc;
   if ((rc = trx_model_reset(h))) return rc;
   if ((rc = trx_model_set_prompt(h, tokens, n, 0))) return rc;
+  if ((rc = check_loaded(m))) return rc;
   // All positions but the last through the batched prefill and a GEMM of the head, unless the sampler
-  // draws at every position or a shape is one that only the single-position kernels take. The last
-  // position leaves the logits and the other outputs of a forward.
+  // draws at every position, a shape is one that only the single-position kernels take, or there is no
+  // room for the batch's buffers. The last position leaves the logits and the other outputs of a forward.
   int done = 0;
-  if (n > 1 && !m.sampling && score_batched(m, n - 1, nll != nullptr) == TRX_OK) {
-    done = n - 1;
-  } else if (n > 1 && !m.sampling) {
-    (void)hipGetLastError();
-    if ((rc = trx_model_reset(h))) return rc;
-    if ((rc = trx_model_set_prompt(h, tokens, n, 0))) return rc;
+  if (n > 1 && !m.sampling && score_takes(m)) {
+    rc = score_alloc(m, n - 1, nll != nullptr);
+    if (rc == TRX_OK) {
+      if ((rc = score_batched(m, n - 1, nll != nullptr))) return rc;
+      done = n - 1;
+    } else if (rc != TRX_E_NOMEM) {
+      return rc;
+    }
   }
   // The captured graph has no score launch, so these positions run eagerly.
   m.scoring = true;

@@ -114,6 +114,8 @@ struct AttnPrefillParams {
   int p0, R, n_head, n_kv, hd, max_ctx, gated;
 };
 int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t s);
+// Whether the RoPE, KV and attention passes above take a geometry.
+bool attn_rows_take(int n_head, int n_kv, int hd, int rope_n, int max_ctx);
 
 // Gated DeltaNet over R positions (fastref.py:182-214, golden.py:400-434):
 //   conv rows: conv + SiLU of every position from the raw projections (the window's older rows
@@ -138,6 +140,7 @@ struct DnRowsParams {
   float eps;
 };
 int launch_dn_rows(const DnRowsParams& p, hipStream_t s);
+bool dn_rows_take(int C, int Kc, int nv, int nk, int hk, int hv);
 
 // Control words after a prefill of positions .. p_last: pos = p_last, cur_tok = fed[p_last].
 int launch_prefill_ctl(int* ctl_pos, int* cur_tok, const int* fed, int p_last, hipStream_t s);

@@ -864,12 +864,18 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void attn_prefill_mfma_kern
     }
 }
 
+// A kv head's cache rows lie below the offset the loads use for keys past a block's queries.
+static bool context_takes(int max_ctx, int hd) { return (size_t)max_ctx * hd * 2 < 0x40000000u; }
+
+bool attn_rows_take(int n_head, int n_kv, int hd, int rope_n, int max_ctx) {
+  return n_kv >= 1 && n_head % n_kv == 0 && n_head / n_kv <= 64 && (hd == 64 || hd == 128 || hd == 256) &&
+         rope_n % 2 == 0 && rope_n <= hd && context_takes(max_ctx, hd);
+}
+
 int launch_attn_prefill(const AttnPrefillParams& p, hipStream_t s) {
   TRX_CHECK(p.n_kv >= 1 && p.n_head % p.n_kv == 0 && p.n_head / p.n_kv <= 64 && p.R >= 1 &&
             p.p0 + p.R <= p.max_ctx, TRX_E_INVALID, "prefill attention: bad geometry");
-  // A kv head's cache rows lie below the offset the loads use for keys past a block's queries.
-  TRX_CHECK((size_t)p.max_ctx * p.hd * 2 < 0x40000000u, TRX_E_INVALID, "prefill attention: context %d too long",
-            p.max_ctx);
+  TRX_CHECK(context_takes(p.max_ctx, p.hd), TRX_E_INVALID, "prefill attention: context %d too long", p.max_ctx);
   const int rep = p.n_head / p.n_kv, QT = 64 / rep;
   if ((p.hd == 64 || p.hd == 128 || p.hd == 256) && rep <= 32) {
     const dim3 mgrid(cdiv(p.R, 4 * (32 / rep)), p.n_kv);
@@ -1081,10 +1087,13 @@ __global__ __launch_bounds__(256) void dn_gnorm_rows_kernel(DnRowsParams p) {
   for (int i = lane; i < hv; i += 64) out[i] = o[i] * rr * p.norm_w[i] * silu(z[i]);
 }
 
+bool dn_rows_take(int C, int Kc, int nv, int nk, int hk, int hv) {
+  return (hk == 64 || hk == 128) && C % hk == 0 && Kc >= 1 && Kc <= 9 && nv % nk == 0 && hv % (hk == 128 ? 8 : 16) == 0 &&
+         hv <= 1024;
+}
+
 int launch_dn_rows(const DnRowsParams& p, hipStream_t s) {
-  const int rb = p.hk == 128 ? 8 : 16;
-  TRX_CHECK(p.R >= 1 && p.R <= kScanRMax && p.hk <= 256 && p.C % p.hk == 0 && p.Kc >= 1 && p.Kc <= 9 &&
-            p.nv % p.nk == 0 && (p.hk == 64 || p.hk == 128) && p.hv % rb == 0 && p.hv <= 1024, TRX_E_INVALID,
+  TRX_CHECK(p.R >= 1 && p.R <= kScanRMax && dn_rows_take(p.C, p.Kc, p.nv, p.nk, p.hk, p.hv), TRX_E_INVALID,
             "prefill DeltaNet: unsupported geometry hk=%d hv=%d Kc=%d (chunk %d)", p.hk, p.hv, p.Kc, p.R);
   hipLaunchKernelGGL(dn_conv_rows_kernel, dim3(p.C / p.hk, cdiv(p.R, kConvRows)), dim3(p.hk), 0, s, p);
   TRX_LAUNCHED();
