@@ -6,7 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from trixium_amd import _lib, configs as C, layout as L
+from trixium_amd import _lib, bons, configs as C, layout as L
 from trixium_amd import synth
 from trixium_amd.model import Decoder, make_config
 
@@ -61,4 +61,18 @@ def test_kv_pin_holds_through_a_score():
         dec.set_kv_ring(1, pin)
         dec.score(toks)
         assert dec.kv_pin == pin
+    dec.close()
+
+
+def test_nan_logit_shows():
+    """One vocabulary row whose scale is NaN: every position's logits hold one, and no NLL hides it."""
+    mc = C.TINY.replace(vocab=1000)
+    dec = Decoder.synthetic(mc, seed=5)
+    rng = np.random.default_rng(5)
+    codes = rng.integers(0, 3, (mc.vocab, mc.n_embd)).astype(np.uint8)
+    scales = rng.uniform(0.01, 0.05, (mc.vocab, mc.n_embd // 128)).astype(np.float16)
+    scales[777, 1] = np.nan
+    dec.set_tensor(L.ROLE_TOK_EMB, 0, bons.encode_rows(L.KIND_TERNARY5, mc.n_embd, scales, codes))
+    nll, _ = dec.score(rng.integers(0, 700, 20))
+    assert np.isnan(nll).all()
     dec.close()

@@ -697,14 +697,18 @@ __global__ __launch_bounds__(1024) void nll_rows_kernel(ScoreRowsParams p) {
       v[k] = i0 + 1024 * k < p.vocab ? lg[i0 + 1024 * k] : -INFINITY;
       top = fmaxf(top, v[k]);
     }
-    if (top == -INFINITY) continue;
+    if (top == -INFINITY) {                           // nothing, or NaN (which no maximum shows)
+#pragma unroll
+      for (int k = 0; k < U; ++k) s += isnan(v[k]) ? v[k] : 0.f;
+      continue;
+    }
     s *= expf(m - top);
 #pragma unroll
     for (int k = 0; k < U; ++k) s += expf(v[k] - top);
     m = top;
   }
   const float wm = wave_max(m);
-  s = wave_sum(m == -INFINITY ? 0.f : s * expf(m - wm));
+  s = wave_sum(m == -INFINITY ? s : s * expf(m - wm));   // s is 0 there, or NaN
   if (lane == 0) {
     rm[tid >> 6] = wm;
     rs[tid >> 6] = s;
@@ -713,7 +717,7 @@ __global__ __launch_bounds__(1024) void nll_rows_kernel(ScoreRowsParams p) {
   if (tid) return;
   float bm = rm[0], t = 0.f;
   for (int i = 1; i < 16; ++i) bm = fmaxf(bm, rm[i]);
-  for (int i = 0; i < 16; ++i) t += rm[i] == -INFINITY ? 0.f : rs[i] * expf(rm[i] - bm);
+  for (int i = 0; i < 16; ++i) t += rm[i] == -INFINITY ? rs[i] : rs[i] * expf(rm[i] - bm);
   p.nll[r] = (bm + logf(t)) - lg[p.target[r]];
 }
 
