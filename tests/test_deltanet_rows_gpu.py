@@ -35,3 +35,32 @@ def test_conv_windows_and_ragged_chunks(tmp_path, kc):
             print("conv", kc, "chunk", chunk, "prefilled", n - 1, "err", err)
             assert err <= 2e-3
         dec.close()
+
+
+def test_longest_chunk():
+    """The longest chunk of a context that the decode attention takes, 8191 positions, against chunks of 512."""
+    from trixium_amd.model import Decoder
+    mc = C.TINY_HYBRID.replace(max_ctx=8192)
+    toks = synth.random_prompt(mc, 8192, 2)
+    out = []
+    for chunk in (512, 8191):
+        dec = Decoder.synthetic(mc, seed=2, prefill_chunk=chunk)
+        out.append(dec.forward(toks).astype(np.float64))
+        dec.close()
+    assert np.max(np.abs(out[1] - out[0])) <= 2e-3 * np.max(np.abs(out[0]))
+
+
+def test_value_heads_of_half_a_block(tmp_path):
+    """Key heads of 128 with value heads of 8 rows: half of the scan's block of 16 rows is empty."""
+    from trixium_amd.model import Decoder
+    cfg = C.TINY_HYBRID.replace(name="tiny-hybrid-hv8", dn_k_head_dim=128, dn_v_head_dim=8, dn_num_v_heads=16)
+    p = str(tmp_path / "c.img")
+    bons.write_image(cfg, synth.small_model_tensors(cfg, 7, True), 1, p, trit5=True)
+    ref = FloatRef(bons.BONSReader(p), kv_fp16=True)
+    tokens = [int(t) for t in np.random.default_rng(7).integers(1, cfg.vocab, 60)]
+    dec = Decoder.from_image(p, prefill_chunk=25)
+    got = dec.forward(tokens)
+    for i, t in enumerate(tokens):
+        want = ref.step(t, want_logits=i == len(tokens) - 1)
+    assert np.max(np.abs(got - want)) <= 2e-3 * np.max(np.abs(want))
+    dec.close()

@@ -963,21 +963,22 @@ __global__ void dn_conv_tail_kernel(DnRowsParams p) {
 }
 
 // The recurrence of one value head over the chunk: 16 state rows per block of 256 threads, a row's HK
-// columns over 16 lanes, row sums by DPP. First every block computes its head's decay and beta gates
-// of all the chunk's positions at once (into LDS), so the serial loop carries only the state's
+// columns over 16 lanes, row sums by DPP. Every block computes its head's decay and beta gates of
+// kScanGates positions at a time (into LDS), so the serial loop carries only the state's
 // arithmetic; k, q and v come through LDS, kScanTile positions at a time, the next tile's loads in
 // flight meanwhile. The per-position arithmetic is dn_recur_fixed_kernel's.
 // Bound by vector issue: the 6144 rows of the 27B shape are 1536 waves of ~50 operations a position.
 // With 32 lanes a row (8 rows a block, two lane swaps a position through LDS, k and q loaded by every
 // wave) a 1024-position chunk took 558 us; 212 us this way.
 constexpr int kScanTile = 16;
-constexpr int kScanRMax = 8192;        // chunk positions whose gates fit the LDS (64 KB)
+constexpr int kScanGates = 2048;       // 16 KB of 50 a block
+constexpr int kScanRMax = 8192;        // chunk positions
 constexpr int kScanRows = 16;
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 template <int HK>
 __global__ __launch_bounds__(256) void dn_scan_kernel(DnRowsParams p) {
   constexpr int V = HK / 64;            // float4s of a row per lane: columns 4 c + 64 i
-  extern __shared__ float2 gates[];     // decay and beta of whole tiles' positions
+  __shared__ float2 gates[kScanGates];  // decay and beta
   __shared__ __align__(16) float kq[2][kScanTile][2 * HK];
   __shared__ float vs[2][kScanTile][kScanRows];
   const int h = blockIdx.x, rb = blockIdx.y, t = threadIdx.x, c = t & 15, tr = t >> 4;
@@ -990,15 +991,19 @@ __global__ __launch_bounds__(256) void dn_scan_kernel(DnRowsParams p) {
   for (int i = 0; i < V; ++i) s[i] = S[16 * i];
   const float Ah = p.A[h], dth = p.dt[h];
   // Positions past the last leave the state as it is.
-  for (int r = t; r < (p.R + kScanTile - 1) / kScanTile * kScanTile; r += 256) {
-    float2 g = make_float2(1.f, 0.f);
-    if (r < p.R) {
-      const float a = p.ba[(size_t)r * 2 * p.nv + p.nv + h] + dth;
-      const float sp = a > 20.f ? a : log1pf(expf(a));
-      g = make_float2(expf(sp * Ah), sigmoidf_(p.ba[(size_t)r * 2 * p.nv + h]));
+  auto fill_gates = [&](int r0) {
+    for (int i = t; i < kScanGates && r0 + i < (p.R + kScanTile - 1) / kScanTile * kScanTile; i += 256) {
+      const int r = r0 + i;
+      float2 g = make_float2(1.f, 0.f);
+      if (r < p.R) {
+        const float a = p.ba[(size_t)r * 2 * p.nv + p.nv + h] + dth;
+        const float sp = a > 20.f ? a : log1pf(expf(a));
+        g = make_float2(expf(sp * Ah), sigmoidf_(p.ba[(size_t)r * 2 * p.nv + h]));
+      }
+      gates[i] = g;
     }
-    gates[r] = g;
-  }
+  };
+  fill_gates(0);
   // Thread (tr, c) stages position tr of a tile: its pieces of k and q, and v of the block's row c.
   f32x4_t kn[V], qn[V];
   float vn;
@@ -1027,10 +1032,14 @@ __global__ __launch_bounds__(256) void dn_scan_kernel(DnRowsParams p) {
   load(kScanTile);
   __syncthreads();
   for (int r0 = 0, buf = 0; r0 < p.R; r0 += kScanTile, buf ^= 1) {
+    if (r0 && r0 % kScanGates == 0) {                  // the last ones are read by nobody past the last barrier
+      fill_gates(r0);
+      __syncthreads();
+    }
     float keep = 0.f;
 #pragma unroll
     for (int u = 0; u < kScanTile; ++u) {
-      const float2 g = gates[r0 + u];
+      const float2 g = gates[r0 % kScanGates + u];
       const float decay = g.x, beta = g.y, vj = vs[buf][u][tr];
       f32x4_t k[V], q[V];
 #pragma unroll
@@ -1102,9 +1111,8 @@ int launch_dn_rows(const DnRowsParams& p, hipStream_t s) {
     TRX_LAUNCHED();
   }
   const dim3 sg(p.nv, cdiv(p.hv, kScanRows));
-  const size_t lds = (size_t)cdiv(p.R, kScanTile) * kScanTile * sizeof(float2);
-  if (p.hk == 128) hipLaunchKernelGGL(dn_scan_kernel<128>, sg, dim3(256), lds, s, p);
-  else hipLaunchKernelGGL(dn_scan_kernel<64>, sg, dim3(256), lds, s, p);
+  if (p.hk == 128) hipLaunchKernelGGL(dn_scan_kernel<128>, sg, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL(dn_scan_kernel<64>, sg, dim3(256), 0, s, p);
   TRX_LAUNCHED();
   hipLaunchKernelGGL(dn_gnorm_rows_kernel, dim3(cdiv(p.nv * p.R, 4)), dim3(256), 0, s, p);
   TRX_LAUNCHED();
