@@ -66,3 +66,22 @@ def test_one_vector_at_any_byte(kind, offset):
     got, status = _call(encode_rows(kind, K, scales, codes), kind, M, K, x8, 27, 10, offset)
     want, wst = _want(codes, scales, x8, 27, 10)
     assert np.array_equal(got, want) and status == wst
+
+
+@pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
+def test_one_vector_of_many_rows(kind):
+    """2^28 weights through the multi-row entry point: one vector takes the single-vector kernel."""
+    rng = np.random.default_rng(kind)
+    K, part, M = 128, 256, 1 << 21
+    codes = rng.integers(0, 3, (part, K)).astype(np.uint8)
+    scales = rng.uniform(0.01, 0.05, (part, 1)).astype(np.float16)
+    x8 = rng.integers(-128, 128, (1, K)).astype(np.int8)
+    rows = np.tile(encode_rows(kind, K, scales, codes).reshape(part, -1), (M // part, 1))
+    rb, xb = _lib.DeviceBuffer(rows.nbytes + 64), _lib.DeviceBuffer.from_array(x8)
+    rb.upload(rows)
+    yb, st = _lib.DeviceBuffer(4 * M), _lib.DeviceBuffer.from_array(np.zeros(1, np.int32))
+    _lib.call("trx_gemv_ternary_exact_rows", rb.ptr, kind, M, K, xb.ptr, 1, 27, 10, yb.ptr, st.ptr, None)
+    _lib.synchronize()
+    want, wst = _want(codes, scales, x8, 27, 10)
+    assert np.array_equal(yb.download(np.int32, M).reshape(M // part, part), np.tile(want, (M // part, 1)))
+    assert int(st.download(np.int32)[0]) == wst

@@ -142,8 +142,7 @@ int gemv_exact_any(const uint8_t* rows, int kind, int M, int K, const int8_t* x8
   const RowGeom rg = row_geom(kind, K);
   RowsParams p = {};
   p.W = rows;
-  // The last group of a row may be read up to 16 bytes past its end: the tensor is followed by a
-  // readable 32-byte tail.
+  // A row's last read ends with its padding at the latest (26 bytes a group, padded to 32).
   p.w_bytes = (uint32_t)((unsigned long long)M * rg.row_bytes + 32);
   p.x8 = x8;
   p.y = y;
@@ -159,6 +158,9 @@ int gemv_exact_any(const uint8_t* rows, int kind, int M, int K, const int8_t* x8
   return kind == TRX_KIND_TERNARY5 ? dispatch_rows<TRX_KIND_TERNARY5>(p, s) : dispatch_rows<TRX_KIND_TERNARY>(p, s);
 }
 
+int gemv_exact(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int B, int R,
+               int32_t* y, int32_t* status, hipStream_t s);
+
 int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, int n, int B,
                     int R, int32_t* y, int32_t* status, hipStream_t s) {
   TRX_CHECK(rows && x8 && y && status, TRX_E_INVALID, "gemv_exact_rows: null argument");
@@ -168,6 +170,9 @@ int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x
   TRX_CHECK((long long)n * K <= kRowsStaged, TRX_E_INVALID,
             "gemv_exact_rows: %d x rows of K=%d exceed %d staged bytes", n, K, kRowsStaged);
   TRX_CHECK(((uintptr_t)x8 & 15) == 0, TRX_E_INVALID, "gemv_exact_rows: x8 must be 16-byte aligned");
+  // One vector of a vocabulary's size: the single-vector kernel's resident blocks (151936 x 4096 44.5 us trit5
+  // and 47.8 2-bit against 70.8 and 61.5 here; 34816 x 5120 24.6 and 20.5 against 23.6 and 21.1).
+  if (n == 1 && (long long)M * K >= (1ll << 28)) return gemv_exact(rows, kind, M, K, x8, B, R, y, status, s);
   return gemv_exact_any(rows, kind, M, K, x8, n, B, R, y, status, s);
 }
 
