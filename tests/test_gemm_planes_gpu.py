@@ -220,3 +220,23 @@ def test_few_values_among_zeros():
     silent = np.zeros(512, bool)
     silent[5] = True
     _check(L.KIND_TERNARY5, 200, 512, 40, _lib.EPI_STORE, False, x, rng, top=np.ones(x.shape), silent=silent)
+
+
+def test_planes_past_4_gib():
+    """Four positions of 2^28 columns: their planes are past what 32-bit offsets reach. Weights of 1, a few columns of
+    x set."""
+    n, K, M, G = 4, 1 << 28, 2, 1 << 21
+    row = np.concatenate([np.full(G, 1, np.float16).view(np.uint8), np.full(32 * G, 0xAA, np.uint8)])
+    rb = _lib.DeviceBuffer.from_array(np.concatenate([row] * M))
+    xb, wb, yb = _lib.DeviceBuffer(4 * n * K), _lib.DeviceBuffer(4 * n * (K + 1)), _lib.DeviceBuffer(4 * n * M)
+    _lib.call("trx_memset_d8", xb.ptr, 0, 4 * n * K, None)
+    want = np.zeros(n)
+    for r in range(n):
+        for i, c in enumerate((5, K // 3, K // 2 + 70, K - 1)):
+            v = np.array([(r + 1) * 1.5 + i], np.float32)
+            xb.upload(v, offset=4 * (r * K + c))
+            want[r] += float(v[0])
+    _lib.call("trx_gemm_ternary_f32", rb.ptr, L.KIND_TERNARY, M, K, xb.ptr, n, None, ctypes.c_float(EPS), yb.ptr,
+              _lib.EPI_STORE, wb.ptr, None)
+    _lib.synchronize()
+    assert np.array_equal(yb.download(np.float32, n * M).reshape(n, M), np.repeat(want[:, None], M, 1))

@@ -254,13 +254,16 @@ struct PlaneReader {
   __amdgpu_buffer_rsrc_t r;
   uint32_t v;                          // this lane's offset in a run of pieces
   uint32_t P;
-  __device__ __forceinline__ void init(const GemmParams& p, int pt, int lane) {
+  int st0;
+  // Steps st0 .. st1 - 1: below 4 GiB of them (the offsets' range).
+  __device__ __forceinline__ void init(const GemmParams& p, int pt, int lane, int st0_, int st1) {
     P = (uint32_t)min(32, p.R - 32 * pt);
+    st0 = st0_;
     const uint32_t j = min((uint32_t)(lane & 31), P - 1), h = (uint32_t)(lane >> 5);
-    r = make_rsrc(p.xp + (size_t)32 * pt * p.K * 4, 4u * P * (uint32_t)p.K);
+    r = make_rsrc(p.xp + ((size_t)32 * pt * p.K * 4 + (size_t)256 * P * st0), 256u * P * (uint32_t)(st1 - st0));
     v = 16u * (h * P + j);
   }
-  __device__ __forceinline__ uint32_t base(int st) const { return 256u * P * (uint32_t)st; }
+  __device__ __forceinline__ uint32_t base(int st) const { return 256u * P * (uint32_t)(st - st0); }
   __device__ __forceinline__ i32x4_t piece(uint32_t base, uint32_t q) const {
     return __builtin_bit_cast(i32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, base + 32u * P * q, 0));
   }
@@ -440,7 +443,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
   RowReader<KIND> row[ND];
   Codes codes[ND], next[ND];                          // the next group's, and the one after
   PlaneReader pl;
-  pl.init(p, pt, lane);
+  pl.init(p, pt, lane, 0, 2 * G);
 #pragma unroll
   for (int d = 0; d < ND; ++d) {
     row[d].init(p, tile_row<EPI>(NT * bx + 4 * d + w, j, p.M), h);
@@ -667,9 +670,9 @@ __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p)
 #pragma unroll
   for (int b = 0; b < NB; ++b) row[b].init(p, tile_row<EPI>(NB * bx + b, j, p.M), h);
   PlaneReader pl;
-  pl.init(p, pt, lane);
-  Codes codes[NB];
   const int gf = min(g0, G - 1);
+  pl.init(p, pt, lane, 2 * gf, 2 * max(g1, gf + 1));
+  Codes codes[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) row[b].load(codes[b], gf);
   Planes q0 = pl.load(2 * gf), q1 = pl.load(2 * gf + 1);
@@ -847,12 +850,13 @@ int launch_gemm_ternary(const GemmParams& params, hipStream_t s) {
   const int tiles = p.epi == GM_SWIGLU ? 2 * cdiv(p.M / 2, 32) : cdiv(p.M, 32), npt = cdiv(p.R, 32);
   const float len[4] = {2.55f, 0.65f, 0.43f, 0.34f};
   const int per[4] = {8, 4, 2, 1};
-  int nb = 0;
+  int nb = -1;
   float best = 0.f;
-  for (int i = 0; i < (p.epi == GM_SWIGLU ? 3 : 4); ++i) {
+  const bool far = (size_t)min(p.R, 32) * p.K * 4 >= (1ull << 32);   // a whole tile's planes: K-split only
+  for (int i = far ? 1 : 0; i < (p.epi == GM_SWIGLU ? 3 : 4); ++i) {
     const long long blocks = (long long)cdiv(tiles, per[i]) * (i == 0 ? cdiv(p.R, 128) : npt);
     const float t = len[i] * (float)((blocks + cus - 1) / cus);
-    if (i == 0 || t < best) {
+    if (nb < 0 || t < best) {
       best = t;
       nb = i == 0 ? 0 : per[i];
     }
