@@ -410,10 +410,10 @@ __device__ __forceinline__ void in_turn(F f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, I>()), ...);
 }
 
-// Large products: a block takes 128 positions x 32 NT weight rows, four waves of one position tile
-// each, one wave a SIMD, so that a wave has 512 registers: NT accumulator tiles, the sums of two pairs
+// Large products: a block takes 128 positions x 256 weight rows, four waves of one position tile
+// each, one wave a SIMD, so that a wave has 512 registers: eight accumulator tiles, the sums of two pairs
 // of tiles and two groups of its positions' planes, which it loads straight into registers a group
-// ahead of their use (the operand order makes each load contiguous). Each wave decodes NT / 4 of the block's
+// ahead of their use (the operand order makes each load contiguous). Each wave decodes two of the block's
 // weight tiles per group into LDS for all, two buffers, one barrier a group.
 // A wave alone issues a vector operation every 6 cycles beside the matrix unit's 32-cycle products,
 // so all other work (the last pair's sums into the accumulators, the next group's decode, the loads)
@@ -424,9 +424,9 @@ __device__ __forceinline__ void in_turn(F f, std::integer_sequence<int, I...>) {
 // group ahead. 2048 positions, planes included: 24576 x 4096 with SwiGLU 503 us (520), 4096 x 12288 with the
 // residual 300 (333); 1024 of 34816 x 5120 491 (521). Per group and round 2.1 to 2.5 us, against 1.75 for the
 // products alone at the power-limited clock.
-template <int KIND, int EPI, int NT>
+template <int KIND, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
-  constexpr int ND = NT / 4, NP = NT / 2;             // tiles a wave decodes, pairs
+  constexpr int NT = 8, ND = NT / 4, NP = NT / 2;     // weight tiles, of them a wave decodes, pairs
   static_assert(NP % 2 == 0, "the pairs take turns with two sets of registers");
   __shared__ __align__(16) uint32_t lut[kLut];
   __shared__ __align__(16) i32x4_t bs[2][NT][2][64];
@@ -807,7 +807,7 @@ static void gemm_ternary_kind(GemmParams& p, int nb, hipStream_t s) {
   if (nb == 0) {
     p.nx = cdiv(tiles, 8);
     p.ny = cdiv(p.R, 128);
-    hipLaunchKernelGGL((gemm_kernel<KIND, EPI, 8>), dim3(p.nx * p.ny), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_kernel<KIND, EPI>), dim3(p.nx * p.ny), dim3(256), 0, s, p);
     return;
   }
   p.nx = cdiv(tiles, nb);

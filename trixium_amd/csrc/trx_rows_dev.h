@@ -101,17 +101,6 @@ struct RowReader {
 #pragma unroll
     for (int i = a; i < b; ++i) v.p[i] = t[((v.d[i >> 2] >> (8 * (i & 3))) & 0xFFu) * 32u];
   }
-  // Holds the uses of the first (second) half's table values behind this point.
-  template <int HALF>
-  __device__ __forceinline__ void ready(Half& v) const {
-    uint32_t* p = v.p;
-    if constexpr (HALF == 0) {
-      asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7]));
-    } else {
-      asm volatile("" : "+v"(p[8]), "+v"(p[9]), "+v"(p[10]), "+v"(p[11]), "+v"(p[12]));
-      if constexpr (KIND == TRX_KIND_TERNARY) asm volatile("" : "+v"(p[13]), "+v"(p[14]), "+v"(p[15]));
-    }
-  }
   __device__ __forceinline__ i32x4_t low(const Half& v) const {
     const uint32_t* p = v.p;
     if (KIND == TRX_KIND_TERNARY5)
