@@ -70,9 +70,9 @@ def test_one_vector_at_any_byte(kind, offset):
 
 @pytest.mark.parametrize("kind", [L.KIND_TERNARY5, L.KIND_TERNARY])
 def test_one_vector_of_many_rows(kind):
-    """2^28 weights through the multi-row entry point: one vector takes the single-vector kernel."""
+    """A large matrix through the multi-row entry point: one vector takes the single-vector kernel."""
     rng = np.random.default_rng(kind)
-    K, part, M = 128, 256, 1 << 21
+    K, part, M = 128, 256, 1 << 18                   # 2^25 weights, rounds of 4096 rows full
     codes = rng.integers(0, 3, (part, K)).astype(np.uint8)
     scales = rng.uniform(0.01, 0.05, (part, 1)).astype(np.float16)
     x8 = rng.integers(-128, 128, (1, K)).astype(np.int8)

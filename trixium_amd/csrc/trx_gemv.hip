@@ -158,8 +158,9 @@ int gemv_exact(const uint8_t* rows, int kind, int M, int K, const int8_t* x8, in
   TRX_CHECK(x8 && y && status, TRX_E_INVALID, "gemv_exact: null argument");
   // The matrix-core kernel (trx_gemv_rows.hip) below 2^25 weights, where its split of K over the waves and
   // its small blocks win (6144 x 2048 7.3 -> 5.1 us, 2048 x 6144 2-bit 9.1 -> 6.0, 4096 x 4096 7.3 ->
-  // 5.8); above, this file's resident blocks (4096 x 12288 2-bit 9.95 against 10.5, 24576 x 4096 12.9
-  // against 13.9, 151936 x 4096 47.6 against 74.6).
+  // 5.8); above, this file's resident blocks (weights from memory: 4096 x 12288 2-bit 10.8 against 13.0,
+  // 24576 x 4096 14.2 against 14.9, 151936 x 4096 49.8 against 82; not where the last round of rows is
+  // nearly empty, 5120 x 17408 28.6 against 20.1).
   if ((long long)M * K < (1ll << 25)) return gemv_exact_any(rows, kind, M, K, x8, 1, B, R, y, status, s);
   TRX_CHECK(B >= -48 && B <= 48 && R >= 0 && R < 63, TRX_E_INVALID, "gemv_exact: B=%d R=%d out of range", B, R);
   GemvParams p = {};

@@ -170,9 +170,13 @@ int gemv_exact_rows(const uint8_t* rows, int kind, int M, int K, const int8_t* x
   TRX_CHECK((long long)n * K <= kRowsStaged, TRX_E_INVALID,
             "gemv_exact_rows: %d x rows of K=%d exceed %d staged bytes", n, K, kRowsStaged);
   TRX_CHECK(((uintptr_t)x8 & 15) == 0, TRX_E_INVALID, "gemv_exact_rows: x8 must be 16-byte aligned");
-  // One vector of a vocabulary's size: the single-vector kernel's resident blocks (151936 x 4096 44.5 us trit5
-  // and 47.8 2-bit against 70.8 and 61.5 here; 34816 x 5120 24.6 and 20.5 against 23.6 and 21.1).
-  if (n == 1 && (long long)M * K >= (1ll << 28)) return gemv_exact(rows, kind, M, K, x8, B, R, y, status, s);
+  // One vector of a large matrix: the single-vector kernel's resident blocks, where their rounds of 4096 rows are
+  // nearly full. Weights from memory, trit5 and 2-bit, us there against here: 151936 x 4096 49.8 and 49.9 against
+  // 82 and 75, 34816 x 5120 25.6 and 21.4 against 26.9 and 26.6, 4096 x 12288 13.0 and 10.8 against 14.7 and
+  // 13.0; with a round of 1024 rows, 5120 x 17408 28.6 and 22.3 against 20.1 and 18.2.
+  const int rounds = cdiv(M, 4096);
+  if (n == 1 && (long long)M * K >= (1ll << 25) && M >= rounds * 3584)
+    return gemv_exact(rows, kind, M, K, x8, B, R, y, status, s);
   return gemv_exact_any(rows, kind, M, K, x8, n, B, R, y, status, s);
 }
 
