@@ -389,8 +389,8 @@ int trx_model_read(trx_model* m, int what, void* host, size_t bytes);
  * prefill, up to 1024 at a time, and a product with the LM head over 128 at a time. Its buffers
  * (those of trx_model_prefill and 128 * vocab floats) stay until the model is destroyed. With the
  * sampler on, which draws at every position, with a head in another format than the layers or a
- * shape that the batched kernels do not take, or without room for the buffers: one position per
- * forward. */
+ * shape that the batched kernels do not take, without room for the buffers, or with fewer than four
+ * tokens: one position per forward. */
 int trx_model_score(trx_model* m, const int32_t* tokens, int n, float* nll, float* hidden);
 /* The LM head applied to n given hidden states (host float32 [n][n_embd] -> [n][vocab]):
  * model/fastref.py:260-261 logits (the rotation of a rotated model included, no norm).

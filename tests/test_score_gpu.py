@@ -17,9 +17,9 @@ def _rel_err(got, ref):
     return float(np.max(np.abs(np.asarray(got, np.float64) - ref)) / np.max(np.abs(ref)))
 
 
-# One and two tokens, one and two of the head's blocks of 128 positions with remainders; a rotated model.
+# One and two tokens, three and four (the fewest that are batched), one and two of the head's blocks of 128 positions with remainders; a rotated model.
 @pytest.mark.parametrize("mc,rot", [(C.TINY, 0), (C.TINY_HYBRID, 0), (C.TINY, 128)])
-@pytest.mark.parametrize("n", [1, 2, 128, 129, 300])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 128, 129, 300])
 def test_score_matches_forwards(mc, rot, n):
     mc = mc.replace(max_ctx=320)
     toks = synth.random_prompt(mc, n, n)
