@@ -13,7 +13,7 @@
 // pair of fp16 values has (root mean square 2.2e-8 against 4.5e-8 for normal x; the last digit at 2^20 and the
 // largest |x| in [8, 16) * 2^u: 6.6e-8). A group's sum is then multiplied by the group's fp16 scale and added in fp32.
 // Measured on all CUs (operands in registers, random data): 6.1 PFLOP/s for fp6 x fp4, 3.4 for
-// int8, 1.57 for fp16; with the planes that each needs for fp32-accurate x (5, 3, 2) that is 1.23,
+// int8, 1.57 for fp16; with the planes that each needs for x to about 24 bits (5, 3, 2) that is 1.23,
 // 1.14 and 0.79 PFLOP/s, and the int8 planes' sums would need five vector operations per element
 // and group where these need one.
 
@@ -423,7 +423,8 @@ __device__ __forceinline__ void in_turn(F f, std::integer_sequence<int, I...>) {
 // Eight waves of four tiles each, at two waves a SIMD, read every plane twice as often and had no room for a
 // group ahead. 2048 positions, planes included: 24576 x 4096 with SwiGLU 503 us (520), 4096 x 12288 with the
 // residual 300 (333); 1024 of 34816 x 5120 491 (521). Per group and round 2.1 to 2.5 us, against 1.75 for the
-// products alone at the power-limited clock.
+// products alone at the power-limited clock (a last digit of one bit more draws more power: 489 -> 500 us and
+// 471 -> 480, measured in turn with the digits as they were).
 template <int KIND, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
   constexpr int NT = 8, ND = NT / 4, NP = NT / 2;     // weight tiles, of them a wave decodes, pairs
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel(GemmParams p) {
 // Products whose grid of large tiles would leave the chip idle: a block takes 32 positions x 32 NB
 // weight rows and its eight waves split K, each decoding its own groups' weights in registers; the
 // waves' sums are added through LDS in wave order. Bound by vector issue (each wave decodes for
-// itself) and, on the shortest prompts, by latency: 24 positions of 6144 x 4096 14.6 us with the
+// itself) and, on the shortest prompts, by latency: 24 positions of 6144 x 4096 15.0 us with the
 // planes (69.5 in 24 large fp16 tiles), 509 of 2048 x 6144 40 us (119).
 template <int KIND, int EPI, int NB>
 __global__ __launch_bounds__(kGmThreads, 1) void gemm_split_kernel(GemmParams p) {
