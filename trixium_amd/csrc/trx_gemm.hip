@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void planes_kernel(PlanesParams p) {
   const uint32_t z = ~seen & ~seen >> 1 & ~seen >> 2 & ~seen >> 3 & 0x0FFFFFFFu;    // four empty ones from here
   const int from = z ? __builtin_ctz(z) : 0;
   const uint32_t low = z ? ~0u << (from + 3) << 1 : 0u;
-  const int first = __builtin_ctz(seen & low | 0x80000000u), gap = first - from;
+  const int first = __builtin_ctz((seen & low) | 0x80000000u), gap = first - from;
   int others = low ? count(low) : 0;
   if (first >= 7 && others > 1 && others * gap < 28) {               // how many they are
     asm volatile("" : "+v"(a), "+v"(b));
